@@ -78,6 +78,26 @@ bool skinny_stages(int rows, int N, int K, int fmt, int input_group, int weight_
     return skinny_staging(rows, N, K, fmt, input_group, weight_group, p) > 0;
 }
 
+// The K-sliced tile (gemm_sliced.hip) for a shape: of the tiles whose grid is
+// one round of workgroups (256 CUs), the one with the least operand bytes per
+// workgroup (they pass L2 -> LDS) plus its share of the epilogue; false when
+// every tile needs a second round. Both weights fit 50 random shapes of 65 to
+// 1100 rows (weights from HBM) and pick within 0.4% of the best tile on
+// average, 4% at worst: 1.36 us per 100 KB, 0.24 us per 1000 outputs.
+bool sliced_tile(int rows, int N, int K, qlin_path *p) {
+    long best = LONG_MAX;
+    for (const auto &t : qlin::kSlicedTiles) {
+        const long wgs = ((long(N) + t.channels - 1) / t.channels) *
+                         ((long(rows) + t.tokens - 1) / t.tokens);
+        const long cost = long(K) * (t.channels + t.tokens) * 14 + t.channels * t.tokens * 243;
+        if (wgs <= 256 && cost < best) {
+            best = cost;
+            *p = {QLIN_KIND_SKINNY, t.tokens, t.channels, 1, 8, 3};
+        }
+    }
+    return best != LONG_MAX;
+}
+
 // Path selection for gfx950 (256 CUs, 8 XCDs). Decode shapes stream the
 // weights once through the skinny kernel; larger token counts use the
 // LDS-tiled MFMA GEMM.
@@ -155,7 +175,25 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
         // 4.65 us, o_proj 4.24 -> 3.64 us.
         p.waves = 8;
         p.staged = skinny_staging(rows, N, K, fmt, input_group, weight_group, p);
+        // Weight slabs of two and three blocks (K above 2048) leave no LDS for
+        // the activation tile; there the K-sliced kernel is ahead once its
+        // rows no longer fit two 16-token tiles (down among a decoder layer's
+        // other launches, FP8, M = 57: 2 us less per layer; M = 32 level).
+        // With one block the slab, all of it in flight from the start, stays
+        // ahead (gate_up at M = 57 2 us less per layer than K-sliced).
+        if (rows > 32 && K > 2048 && !input_group && !weight_group) {
+            qlin_path sliced;
+            if (sliced_tile(rows, N, K, &sliced)) return sliced;
+        }
         return p;
+    }
+    // Up to about a thousand rows, grids that a K-sliced tile covers in one
+    // round: 65 shapes of 65-1000 rows measured 1.46x faster on average than
+    // the macro tiles below, the worst 8% slower. From 1024 rows the macro
+    // tiles fill the GPU themselves (o_proj at 1024: 9.4 us on 128x64).
+    if (rows < 1024 && !input_group && !weight_group) {
+        qlin_path sliced;
+        if (sliced_tile(rows, N, K, &sliced)) return sliced;
     }
     // Prefill: the macro tile by measured MI355X rules (BASELINE projections
     // at M = 1024 and 4096, per-channel and K128 groups, realistic data).
@@ -239,6 +277,20 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
 
 int check_path(const qlin_path &p, int rows, int N, int K, int fmt, int input_group,
                int weight_group) {
+    if (p.kind == QLIN_KIND_SKINNY && p.staged == 3) {
+        bool known = false;
+        for (const auto &t : qlin::kSlicedTiles)
+            known = known || (t.channels == p.channels && t.tokens == p.tokens);
+        if (!known || p.waves != 8 || p.splits != 1)
+            return fail(QLIN_ERR_UNSUPPORTED, "no K-sliced %dx%d path (waves %d, splits %d)",
+                        p.channels, p.tokens, p.waves, p.splits);
+        if (input_group || weight_group)
+            return fail(QLIN_ERR_UNSUPPORTED, "K-sliced paths have per-channel scales only");
+        if (((long(N) + p.channels - 1) / p.channels) * ((long(rows) + p.tokens - 1) / p.tokens) >
+            INT32_MAX)
+            return fail(QLIN_ERR_UNSUPPORTED, "K-sliced path has more than 2^31 - 1 macro tiles");
+        return ok();
+    }
     if (p.kind == QLIN_KIND_SKINNY) {
         if (p.tokens != 16 && p.tokens != 32 && p.tokens != 64)
             return fail(QLIN_ERR_UNSUPPORTED, "skinny path tokens must be 16/32/64 (got %d)",
@@ -254,7 +306,7 @@ int check_path(const qlin_path &p, int rows, int N, int K, int fmt, int input_gr
                         "skinny path splits (%d) must be in 1..ceil(K/256) = %d", p.splits,
                         blocks_k);
         if (p.staged < 0 || p.staged > 2)
-            return fail(QLIN_ERR_UNSUPPORTED, "skinny staged must be 0, 1 or 2");
+            return fail(QLIN_ERR_UNSUPPORTED, "skinny staged must be 0, 1, 2 or 3");
         // Token tiles run along the grid's z dimension (at most 65535).
         if ((long(rows) + p.tokens - 1) / p.tokens > 65535)
             return fail(QLIN_ERR_UNSUPPORTED, "skinny path has more than 65535 token tiles");
@@ -419,8 +471,9 @@ int gemm_impl(const qlin_path *path, const void *x, const float *sx, const void 
     if (!aligned(sx, 4) || !aligned(sw, 4))
         return fail(QLIN_ERR_ALIGNMENT, "scales must be 4-byte aligned");
     qlin_path p = path && path->kind ? *path : choose(rows, N, K, fmt, input_group, weight_group);
-    // Packed weights stream straight into registers: no LDS slab staging.
-    if (packed && !(path && path->kind)) p.staged = 0;
+    // Packed weights stream straight into registers: no LDS slab staging (the
+    // K-sliced and prefill kernels stage them like row-major ones).
+    if (packed && !(path && path->kind) && p.staged != 3) p.staged = 0;
     int status = check_path(p, rows, N, K, fmt, input_group, weight_group);
     if (status) return status;
     qlin::GemmArgs a{static_cast<const uint8_t *>(x),
@@ -458,7 +511,9 @@ int gemm_impl(const qlin_path *path, const void *x, const float *sx, const void 
     if (need && !aligned(workspace, 16))
         return fail(QLIN_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    int r = p.kind == QLIN_KIND_SKINNY ? qlin::launch_skinny(a, ip, s) : qlin::launch_tiled(a, ip, s);
+    int r = p.kind != QLIN_KIND_SKINNY ? qlin::launch_tiled(a, ip, s)
+            : p.staged == 3            ? qlin::launch_sliced(a, ip, s)
+                                       : qlin::launch_skinny(a, ip, s);
     if (r) return fail(r, "no kernel variant for this path");
     return check_launch("quantized GEMM launch");
 }

@@ -245,6 +245,15 @@ __device__ __noinline__ void finish4(float (&v)[4], const uint16_t *bias, int n,
     }
 }
 
+// ---------------------------------------------------------------- tile numbering
+// XCD-major numbering of a grid of `tiles` workgroups: the hardware places
+// workgroup i on XCD i % 8, and the tiles that one XCD gets are consecutive
+// (the first tiles % 8 XCDs have one more), so they share its L2.
+__device__ __forceinline__ int xcd_major(int i, int tiles) {
+    const int x = i % 8;
+    return x * (tiles / 8) + min(x, tiles % 8) + i / 8;
+}
+
 // ---------------------------------------------------------------- wave64 reductions
 // The value held by lane (lane ^ S), S a power of two up to 32, without an
 // LDS round trip: S = 1, 2 by a DPP quad permutation, 4 by two row rotations

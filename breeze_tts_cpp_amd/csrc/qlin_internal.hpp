@@ -136,6 +136,13 @@ size_t skinny_lds_bytes(const GemmArgs &, const GemmPath &);
 int skinny_span(int K, int splits);
 constexpr size_t kLdsBytes = 160 * 1024;  // per workgroup on gfx950
 int launch_tiled(const GemmArgs &, const GemmPath &, hipStream_t);
+// K-sliced family (KIND_SKINNY with staged 3; gemm_sliced.hip): per-channel
+// scales, the tiles below (channels x tokens).
+int launch_sliced(const GemmArgs &, const GemmPath &, hipStream_t);
+constexpr struct { int channels, tokens; } kSlicedTiles[] = {
+    {16, 16}, {16, 32}, {16, 48}, {16, 64}, {32, 16}, {32, 32}, {32, 48}, {32, 64}, {32, 80},
+    {48, 32}, {48, 48}, {48, 64}, {48, 80}, {48, 96}, {64, 32}, {64, 48}, {64, 64},
+    {64, 96}, {64, 128}, {96, 64}, {96, 96}};
 // Packed weight layout (weight_pack.hip): N % 16 == 0, bytes = N * ceil(K/64)*64.
 size_t packed_weight_bytes(int N, int K);
 void launch_pack_weights(const void *w, int N, int K, void *packed, hipStream_t);

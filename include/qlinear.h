@@ -75,7 +75,7 @@ enum {
 /* Kernel families (qlin_path.kind). */
 enum {
     QLIN_KIND_AUTO = 0,   /* qlin_gemm plans itself */
-    QLIN_KIND_SKINNY = 1, /* decode regime: weight-streaming MFMA GEMM, tokens <= 64 per tile */
+    QLIN_KIND_SKINNY = 1, /* waves split K: decode, and small grids up to about 1000 tokens */
     QLIN_KIND_TILED = 2   /* prefill regime: LDS-tiled MFMA GEMM */
 };
 
@@ -89,8 +89,10 @@ typedef struct qlin_path {
     int waves;    /* skinny: 8 (wave64s splitting K inside a workgroup);
                      tiled: 1, 2, 4 or 8 (the macro tile's wave layout) */
     int staged;   /* skinny: 1 = each wave's weight slab staged global->LDS
-                     in one shot, 0 = weights loaded straight to registers;
-                     tiled: 0 */
+                     in one shot, 2 = its activation rows too, 0 = weights
+                     loaded straight to registers, 3 = K-sliced: both
+                     operands through per-slice LDS rings (per-channel
+                     scales, its own channel x token tiles); tiled: 0 */
 } qlin_path;
 
 /* Library version (major*10000 + minor*100 + patch). */
@@ -195,8 +197,8 @@ int qlin_pack_weights(const void *w, int N, int K, void *packed, qlin_stream_t s
 
 /* qlin_gemm / qlin_linear with w in the packed layout (same scales, same
  * results bit for bit). Decode paths stream the packed tiles straight into
- * MFMA registers (no LDS staging; path.staged and path.splits > 1 are not
- * supported); prefill paths stage them through LDS like row-major weights. */
+ * MFMA registers (no LDS staging; path.staged 1 / 2 and path.splits > 1 are
+ * not supported); K-sliced and prefill paths stage them through LDS like row-major weights. */
 int qlin_gemm_packed(const qlin_path *path, const void *x, const float *sx, const void *w,
                      const float *sw, void *y, int rows, int N, int K, int fmt, int out_type,
                      int input_group, int weight_group, void *workspace, size_t workspace_bytes,
