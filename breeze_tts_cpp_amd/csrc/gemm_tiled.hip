@@ -27,7 +27,8 @@
 // past the matrix edge and chunks past K read as zero (out-of-range offset).
 // The weight tile is the MFMA A operand: a lane's accumulator holds four
 // consecutive output channels of one token -> 8-byte output stores.
-// Tiles are numbered XCD-major (consecutive tiles on one XCD share its L2).
+// Tiles are numbered XCD-major (consecutive tiles on one XCD share its L2),
+// for any number of tiles.
 #include "qlin_device.hpp"
 #include "qlin_internal.hpp"
 
@@ -112,12 +113,15 @@ __device__ __forceinline__ void store_out16(uint16_t *dst, const uint4 &val) {
                                 reinterpret_cast<i32x4 *>(dst));
 }
 
+constexpr int group_width(int bn, int bm) { return bn == 256 && bm == 256 ? 8 : 4; }
+
 template <int Fmt, int WN, int WM, int WTN, int WTM, int BK, int STAGES, bool Grouped, bool KFull,
           class Out, bool PackedW = false, int GS = 128>
 __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
     const uint8_t *__restrict__ x, const float *__restrict__ sx, const uint8_t *__restrict__ w,
     const float *__restrict__ sw, void *__restrict__ y, int M, int N, int K, int tiles_m,
-    int tiles_n, int input_group, int weight_group, const uint16_t *__restrict__ bias, int act) {
+    int tiles_n, int input_group, int weight_group, const uint16_t *__restrict__ bias, int act,
+    int window) {
     constexpr int NW = WN * WM;
     constexpr int BN = 16 * WTN * WN, BM = 16 * WTM * WM;
     constexpr int CPR = BK / 16;          // 16-byte chunks per stage row
@@ -157,16 +161,13 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
 
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
-    // XCD-major tile numbering: hardware places workgroup b on XCD b % 8.
-    const int tiles = tiles_m * tiles_n;
-    int b = blockIdx.x;
-    if (tiles % 8 == 0) b = (b % 8) * (tiles / 8) + b / 8;
+    const int b = xcd_major(blockIdx.x, tiles_m * tiles_n);
     // Column groups of kGroupN weight tiles: consecutive tiles (one XCD's
     // share) cover a kGroupN x (tiles/8/kGroupN) block, not one tall column.
     // 256x256 tiles take groups of 8 (qkv at M = 4096: INT8 35.1 -> 34.3 us,
     // FP8 33.6 -> 32.5 us, gate_up 0.5% faster); the other tiles groups of 4
     // (8 measured 1% slower on o_proj and down).
-    constexpr int kGroupN = BN == 256 && BM == 256 ? 8 : 4;
+    constexpr int kGroupN = group_width(BN, BM);
     const int group = b / (kGroupN * tiles_m), in_group = b % (kGroupN * tiles_m);
     const int group_w = min(kGroupN, tiles_n - group * kGroupN);
     const int tn = group * kGroupN + in_group % group_w, tm = in_group / group_w;
@@ -221,8 +222,15 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
     const uint32_t scale_stride = scale_groups ? uint32_t((scale_wv ? N : M) * 4) : 0u;
     const uint32_t scale_lane =
         uint32_t((scale_groups ? (scale_wv ? n_base : m_base) * 4 : 0) + lane * 16);
+    // Per channel, the stages of each whole window of `window` (a power of
+    // two) are walked from another start in each workgroup (see turn_window;
+    // 256x256 tiles carry no code for it, which cost them 1-3%).
+    const int stages = (K + BK - 1) / BK;
     auto issue = [&](int stage, int k0) {
         uint8_t *base = lds + (stage % STAGES) * STAGE_BYTES;
+        if constexpr (!Grouped && BM < 256)
+            if ((stage | (window - 1)) < stages)
+                k0 = ((stage & -window) | ((stage + 3 * b) & (window - 1))) * BK;
         const bool kin = KFull || k0 + lane_chunk * 16 < K;
         const uint32_t voff = kin ? lane_voff + uint32_t(k0) : 0x80000000u;
         const uint32_t voff_p = kin ? lane_voff_p : 0x80000000u;
@@ -315,7 +323,6 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
         }
         scale_v[l] = v;
     }
-    const int stages = (K + BK - 1) / BK;
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s)
         if (s < stages) issue(s, s * BK);
@@ -988,9 +995,7 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void wide_gemm(
     static_assert(ROWS % (RPI * NW) == 0 && BN % (RPI * NW) == 0, "stage rows per instruction");
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
-    const int tiles = tiles_m * tiles_n;
-    int b = blockIdx.x;
-    if (tiles % 8 == 0) b = (b % 8) * (tiles / 8) + b / 8;
+    const int b = xcd_major(blockIdx.x, tiles_m * tiles_n);
     constexpr int kGroupN = 4;
     const int group = b / (kGroupN * tiles_m), in_group = b % (kGroupN * tiles_m);
     const int group_w = min(kGroupN, tiles_n - group * kGroupN);
@@ -1237,6 +1242,29 @@ int launch_wide(const GemmArgs &a, hipStream_t stream) {
     return 0;
 }
 
+// Stages per window of a turned K walk (1 = in order). At one K column, rows of
+// a pitch that is a multiple of 1 KB lie on few L2 channels, and workgroups
+// that start together read the same columns at the same time. Starting each
+// at another stage of a window spreads them, as long as a window of the rows
+// that an XCD's workgroups read at once stays in its L2 (4 MB; 4.5 measured
+// as well). us, in order -> turned: qkv at M = 1024 INT8 18.2 -> 14.0, FP8
+// 17.9 -> 13.8, at 730 17.2 -> 12.8; down at 4096 INT8 56.2 -> 54.5, FP8 61.6
+// -> 54.8. Not taken by 256x256 tiles (gate_up at 1024 5% slower), nor by
+// grids past one round unless all of K is one window (gate_up at M = 431 20.2
+// -> 19.4; o_proj at 4096, a window of half of K, 3% slower).
+int turn_window(int K, int BK, int BN, int BM, int tiles_n, int tiles_m) {
+    const long tiles = long(tiles_n) * tiles_m;
+    const int stages = (K + BK - 1) / BK;
+    const int live = int(std::min(64L, (tiles + 7) / 8));
+    const int gn = std::min(group_width(BN, BM), tiles_n);
+    const int gm = std::min(tiles_m, (live + gn - 1) / gn);
+    const long rows = long(std::min(tiles_n, (live + gn * gm - 1) / (gn * gm) * gn)) * BN + long(gm) * BM;
+    const long fit = 4608L * 1024 / (rows * BK);
+    int window = 1;
+    while (window * 2 <= fit && window * 2 <= stages) window *= 2;
+    return BM == 256 || (tiles > 256 && window * 2 <= stages) ? 1 : window;
+}
+
 template <int Fmt, int WN, int WM, int WTN, int WTM, int BK, int STAGES, bool Grouped, class Out,
           int GS = 128>
 int launch_shape(const GemmArgs &a, hipStream_t stream) {
@@ -1245,10 +1273,11 @@ int launch_shape(const GemmArgs &a, hipStream_t stream) {
     const size_t stage = size_t(BN + BM) * BK + (Grouped && GS == 128 ? 3072 : 0);
     const size_t lds = std::max(size_t(STAGES) * stage, size_t(BN) * BM * 2) + size_t(BN + BM) * 4;
     dim3 grid(unsigned(tiles_n * tiles_m)), block(64 * WN * WM);
+    const int window = turn_window(a.K, BK, BN, BM, tiles_n, tiles_m);
 #define QLIN_TILED(KF, PW)                                                                      \
     hipLaunchKernelGGL((tiled_gemm<Fmt, WN, WM, WTN, WTM, BK, STAGES, Grouped, KF, Out, PW, GS>), \
                        grid, block, lds, stream, a.x, a.sx, a.w, a.sw, a.y, a.M, a.N, a.K,      \
-                       tiles_m, tiles_n, a.input_group, a.weight_group, a.bias, a.act)
+                       tiles_m, tiles_n, a.input_group, a.weight_group, a.bias, a.act, window)
     if (a.K % BK == 0) { if (a.packed) QLIN_TILED(true, true); else QLIN_TILED(true, false); }
     else { if (a.packed) QLIN_TILED(false, true); else QLIN_TILED(false, false); }
 #undef QLIN_TILED

@@ -385,3 +385,23 @@ def test_prefill_graph_replay(dev, orc, fmt):
             assert torch.equal(y.view(torch.int16), ref.view(torch.int16)), f"replay {r}"
             qlinear.gemm(*args)  # eager work between replays
         del g
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [I8, FP8])
+@pytest.mark.parametrize("M,N,K", [(300, 400, 2048), (130, 528, 4224), (260, 272, 1040)])
+def test_tiled_turned_walk(dev, orc, fmt, M, N, K):
+    """Grids of one round, whose workgroups walk K from different starts:
+    windows of all of K, of part of it (the last stages in order) and with a
+    partial last stage; a tile count that is no multiple of the eight XCDs;
+    every output row against the oracle."""
+    from breeze_tts_cpp_amd.qlinear import Path, KIND_TILED
+    xq, sx, wq, sw = operands(orc, M, N, K, fmt, seed=M + K)
+    ideal = None if fmt == I8 else orc.gemm_fp8_ideal(xq, sx, wq, sw)
+    for channels, tokens in ((256, 128), (128, 128), (128, 64)):
+        print(f"turned {channels}x{tokens} fmt={fmt} M={M} N={N} K={K}", flush=True)
+        y = gpu_gemm(dev, xq, sx, wq, sw, fmt, path=Path(KIND_TILED, tokens, channels, 1, 8))
+        if fmt == I8:
+            check_i8(orc, y, xq, sx, wq, sw)
+        else:
+            assert rel_l2(bits_to_f32(y), ideal) <= FP8_REL_L2
