@@ -10,8 +10,8 @@
 //     indexed residual, condition, sequence-tail mask, output scale,
 //     activation) -> row quantization (reference pointwise_quantize,
 //     sequence_pointwise.cu:149-260,325-357).
-//   norm_project: LayerNorm -> per-token quantization -> GEMV in one launch,
-//     k <= 512 (reference normalized_quantized_linear, sequence_norm.cu:
+//   norm_project, norm_project_rows: LayerNorm -> per-token quantization ->
+//     GEMV in one launch, one or eight rows per workgroup, k <= 512 (reference normalized_quantized_linear, sequence_norm.cu:
 //     216-390,518-575).
 //
 // One 256-thread workgroup per row. The row quantizers hold the row in
@@ -689,6 +689,289 @@ __global__ __launch_bounds__(256) void norm_project(
     }
 }
 
+// The LayerNorm and quantization of one row by one wave, with the sums of a
+// 256-thread workgroup whose thread t holds columns t and t + 256 (the
+// reference's, see block_sum_256): lane l stands for threads l + 64j, j < 4, so
+// it holds columns l + 64j; each j's 32-lane trees give group totals 2j and
+// 2j + 1, added in group order.
+__device__ __forceinline__ float wave_sum_256(const float (&p)[4]) {
+    float total = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float v = p[j];
+        v += lane_xor<1>(v);
+        v += lane_xor<2>(v);
+        v += lane_xor<4>(v);
+        v += lane_xor<8>(v);
+        v += lane_xor<16>(v);
+        const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
+        const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
+        total = j ? total + lo : lo;
+        total += hi;
+    }
+    return total;
+}
+
+// Eight rows x 128 * reps channels per workgroup of eight waves: each wave
+// LayerNorms and quantizes one row (codes to LDS: INT8 as they are, FP8
+// decoded to the 16-bit type), then takes 16 channels of every 128. Its first
+// weights are requested ahead of the LayerNorm, whose latency covers them.
+// INT8: v_mfma_i32_16x16x64_i8, weights the A operand (16-byte pieces of 16
+// rows, past k multiplied by zero codes), the eight rows half of B. FP8: each
+// 32-lane group takes one channel at a time, its weights decoded once for the
+// eight rows; lane l32 sums words c = 4 l32 + 128 j in order and the 32 lanes
+// reduce as sum32_down, all eight rows in one tree (at distances 16, 8 and 4
+// each exchange carries two rows).
+constexpr int kProjRows = 8, kProjChannels = 128, kProjPitch = 528;
+template <int Fmt, class T>
+__global__ __launch_bounds__(512) void norm_project_rows(
+    const uint16_t *__restrict__ x, qlin_norm_fusion f, const uint16_t *__restrict__ nw,
+    const uint16_t *__restrict__ nb, int rows, int k, float eps, const uint8_t *__restrict__ w,
+    const float *__restrict__ sw, int n, int reps, const uint16_t *__restrict__ bias, int act,
+    uint16_t *__restrict__ y, uint16_t *__restrict__ normalized, uint8_t *__restrict__ encoded,
+    float *__restrict__ encoded_scales) {
+    __shared__ __attribute__((aligned(16))) uint8_t codes[Fmt == I8 ? kProjRows * kProjPitch : 16];
+    __shared__ __attribute__((aligned(16))) float act32[Fmt == I8 ? 4 : kProjRows * 512];
+    __shared__ float steps[kProjRows];
+    __shared__ __attribute__((aligned(8))) uint16_t out[kProjRows * kProjChannels];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int row0 = blockIdx.y * kProjRows, row = row0 + wave;
+    const bool first = blockIdx.x == 0;
+    const int blocks = (n + kProjChannels - 1) / kProjChannels;
+    const int block0 = blockIdx.x * reps, block1 = min(block0 + reps, blocks);
+
+    // INT8: this wave's 16 channels of a block, lane (channel lane % 16,
+    // quad lane / 16) holding K bytes [64 p + 16 quad, +16).
+    // Channels past n read as zeros (the descriptor ends at the last row).
+    const int pieces = (k + 63) / 64;
+    i32x4 wreg[Fmt == I8 ? 8 : 1];
+    float swreg[4];     // of the lane's four output channels
+    uint16_t breg[4];
+    auto load_w = [&](int block) {
+        const int base = block * kProjChannels;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int channel = min(base + wave * 16 + (lane >> 4) * 4 + r, n - 1);
+            swreg[r] = sw[channel];
+            breg[r] = bias ? bias[channel] : uint16_t(0);
+        }
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t *>(w + size_t(base) * k), 0, min(kProjChannels, n - base) * k,
+            0x00020000);
+        const uint32_t off = uint32_t((wave * 16 + (lane & 15)) * k + (lane >> 4) * 16);
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+            if (p < pieces) wreg[p] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + p * 64, 0, 0);
+    };
+    if constexpr (Fmt == I8) load_w(block0);
+
+    if (row < rows) {
+        const int sequence = row / f.rows_per_sequence;
+        const uint16_t *pb = row_of(f.projection_bias, 1, 0, k);
+        const uint16_t *gate = row_of(f.gate, f.gate_rows, sequence, k);
+        const uint16_t *res = row_of(f.residual, rows, row, k);
+        const uint16_t *scale = row_of(f.scale, f.scale_rows, sequence, k);
+        const uint16_t *shift = row_of(f.shift, f.shift_rows, sequence, k);
+        uint16_t *raw = f.raw ? static_cast<uint16_t *>(f.raw) + size_t(row) * k : nullptr;
+        // Every operand is requested before any is used (columns past k read
+        // the last one and are dropped below), so the row waits for memory once.
+        auto fetch = [&](const uint16_t *p, uint16_t (&d)[8], uint16_t absent) {
+            if (p) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d[i] = p[min(lane + i * 64, k - 1)];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d[i] = absent;
+            }
+        };
+        uint16_t xv[8], pbv[8], gv[8], rv[8], wv[8], bv[8], scv[8], shv[8];
+        fetch(x + size_t(row) * k, xv, 0);
+        fetch(pb, pbv, 0);
+        fetch(gate, gv, 0);
+        fetch(res, rv, 0);
+        fetch(nw, wv, 0);
+        fetch(nb, bv, 0);
+        fetch(scale, scv, 0);
+        fetch(shift, shv, 0);
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int c = lane + i * 64;
+            float a = round16<T>(to_float(xv[i], T{}) + to_float(pbv[i], T{}));
+            if (gate) a = round16<T>(a * to_float(gv[i], T{}));
+            a = round16<T>(a + to_float(rv[i], T{}));
+            if (first && raw && c < k) raw[c] = from_float(a, T{});
+            v[i] = c < k ? a : 0.f;
+        }
+        float part[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[j] = (0.f + v[j]) + v[j + 4];
+        const float mean = wave_sum_256(part) / float(k);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float sum = 0.f;
+#pragma unroll
+            for (int i = j; i < 8; i += 4)
+                if (lane + i * 64 < k) {
+                    const float d = v[i] - mean;
+                    sum = __builtin_fmaf(d, d, sum);
+                }
+            part[j] = sum;
+        }
+        const float inv = rsqrt_rn(wave_sum_256(part) / float(k) + eps);
+        float amax = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int c = lane + i * 64;
+            float val = (v[i] - mean) * inv;
+            if (nw) val = val * to_float(wv[i], T{});
+            val = round16<T>(val + to_float(bv[i], T{}));
+            if (scale) val = round16<T>(val * round16<T>(1.f + to_float(scv[i], T{})));
+            val = round16<T>(val + to_float(shv[i], T{}));
+            if (c < k) amax = fmaxf(amax, fabsf(val));
+            if (first && normalized && c < k) normalized[size_t(row) * k + c] = from_float(val, T{});
+            v[i] = val;
+        }
+        const float step = quant_scale<Fmt>(group_max<64>(amax));
+        const float recip = 1.f / step;
+        if (lane == 0) {
+            steps[wave] = step;
+            if (first && encoded_scales) encoded_scales[row] = step;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int c = lane + i * 64;
+            // columns past k hold zero codes
+            const uint32_t code = c < k ? encode<Fmt>(v[i] * recip) : 0u;
+            if constexpr (Fmt == I8) codes[wave * kProjPitch + c] = uint8_t(code);
+            else act32[wave * 512 + c] = round16<T>(decode_fp8(code));
+            if (first && encoded && c < k) encoded[size_t(row) * k + c] = uint8_t(code);
+        }
+    } else if (lane == 0) {
+        steps[wave] = 1.f;  // a row past the end: its products are not stored
+    }
+    __syncthreads();
+
+    // (acc * sw) * step, rounded, bias, ReLU.
+    auto finish = [&](float scaled, uint16_t b) {
+        float o = round16<T>(scaled);
+        o = round16<T>(o + to_float(b, T{}));
+        if (act == FINISH_RELU) o = fmaxf(o, 0.f);
+        return from_float(o, T{});
+    };
+    for (int block = block0; block < block1; ++block) {
+        const int base = block * kProjChannels;
+        if constexpr (Fmt == I8) {
+            const int m = lane & 7;  // B rows 8-15 repeat rows 0-7; their results are dropped
+            const uint8_t *crow = codes + m * kProjPitch + (lane >> 4) * 16;
+            i32x4 acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int p = 0; p < 8; ++p)
+                if (p < pieces)
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                        wreg[p], *reinterpret_cast<const i32x4 *>(crow + p * 64), acc, 0, 0, 0);
+            if ((lane & 15) < kProjRows) {
+                const float step = steps[m];
+                const int c0 = wave * 16 + (lane >> 4) * 4;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    out[m * kProjChannels + c0 + r] =
+                        finish((float(acc[r]) * swreg[r]) * step, breg[r]);
+            }
+            if (block + 1 < block1) load_w(block + 1);
+        } else {
+            const int l32 = t & 31, hi4 = (l32 >> 2) & 7, count = min(kProjRows, rows - row0);
+            const float step = steps[hi4];
+            // Two channels (ch, ch + 16) at a time share the activation reads;
+            // the next two's words are requested under them.
+            uint32_t wq[2][4];
+            float scale_n[2];
+            uint16_t bias_n[2];
+            auto words = [&](int ch) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int channel = min(base + ch + 16 * h, n - 1);
+                    scale_n[h] = sw[channel];
+                    bias_n[h] = bias ? bias[channel] : uint16_t(0);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int c = l32 * 4 + j * 128;
+                        wq[h][j] = c < k ? *reinterpret_cast<const uint32_t *>(
+                                               w + size_t(channel) * k + c)
+                                         : 0u;
+                    }
+                }
+            };
+            words(t >> 5);
+            for (int ch = t >> 5; ch < kProjChannels; ch += 32) {
+                if (base + ch >= n) break;
+                float wf[2][4][4];
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        // exact e4m3fn -> fp32
+                        const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(int(wq[h][j]), false);
+                        const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(int(wq[h][j]), true);
+                        wf[h][j][0] = lo[0], wf[h][j][1] = lo[1];
+                        wf[h][j][2] = hi[0], wf[h][j][3] = hi[1];
+                    }
+                const float scale_c[2] = {scale_n[0], scale_n[1]};
+                const uint16_t bias_c[2] = {bias_n[0], bias_n[1]};
+                if (ch + 32 < kProjChannels) words(ch + 32);
+                float s[2][kProjRows];
+#pragma unroll
+                for (int r = 0; r < kProjRows; ++r) {
+                    s[0][r] = s[1][r] = 0.f;
+                    if (r >= count) continue;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int c = l32 * 4 + j * 128;
+                        if (j * 128 >= k) break;
+                        const f32x4 av = *reinterpret_cast<const f32x4 *>(act32 + r * 512 + c);
+                        // past k both factors are zero: the sum keeps its value
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                s[h][r] = __builtin_fmaf(av[e], wf[h][j][e], s[h][r]);
+                    }
+                }
+                // Distance 16: lanes with bit 16 clear go on with row r, the
+                // others with row r + 4; then 8 (r, r + 2) and 4 (r, r + 1).
+                auto pair = [&](float a, float b, int bit, auto xchg) {
+                    const bool up = l32 & bit;
+                    const float keep = up ? b : a, give = up ? a : b;
+                    return keep + xchg(give);
+                };
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    float q4[4], q2[2];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        q4[r] = pair(s[h][r], s[h][r + 4], 16, [](float z) { return lane_xor<16>(z); });
+#pragma unroll
+                    for (int r = 0; r < 2; ++r)
+                        q2[r] = pair(q4[r], q4[r + 2], 8, [](float z) { return lane_xor<8>(z); });
+                    float q1 = pair(q2[0], q2[1], 4, [](float z) { return lane_xor<4>(z); });
+                    q1 += lane_xor<2>(q1);
+                    q1 += lane_xor<1>(q1);
+                    if ((l32 & 3) == 0)
+                        out[hi4 * kProjChannels + ch + 16 * h] =
+                            finish((q1 * scale_c[h]) * step, bias_c[h]);
+                }
+            }
+        }
+        __syncthreads();
+        for (int i = t; i < kProjRows * kProjChannels; i += 512) {
+            const int m = i / kProjChannels, c = i % kProjChannels;
+            if (row0 + m < rows && base + c < n) y[size_t(row0 + m) * n + base + c] = out[i];
+        }
+        __syncthreads();
+    }
+}
+
 // ---------------------------------------------------------------- launchers
 // The row-quantizer variants (format x 16-bit type x items per lane x
 // vector access) compile in four parallel parts, one
@@ -785,9 +1068,39 @@ void launch_pointwise_quantize(const PointwiseQuantizeArgs &a, hipStream_t strea
 // because a 32-lane group's channels run one after another.
 constexpr int kTargetBlocks = 2048, kMaxReps = 16;
 void launch_norm_linear(const NormLinearArgs &a, hipStream_t stream) {
+    const int blocks8 = (a.n + 7) / 8;
+    // Above about 3000 (FP8: 6000) pairs of a row and eight channels, eight
+    // rows per workgroup: norm_project's time grows with every pair, because
+    // each repeats the row's LayerNorm. us, one row per workgroup -> eight:
+    // INT8, n 2048: 16 rows 8.4 -> 7.8, 32 rows 10.5 -> 7.8, 150 rows 30.6 ->
+    // 10.6, 1500 rows 198 -> 38, but 8 rows 7.5 -> 7.7 and 1 row 4.6 -> 6.7; FP8:
+    // 32 rows 23 -> 16.5, 150 rows 83 -> 22, but 16 rows 15.4 -> 16.4 (bf16, k
+    // 512). Bound by the LayerNorm's dependent sums (about 3 us) and one
+    // round trip for the weights; FP8 by its fp32 products.
+    if (int64_t(blocks8) * a.rows >= (a.fmt == I8 ? 3072 : 6144)) {
+        const int blocks = (a.n + kProjChannels - 1) / kProjChannels;
+        const int tiles = (a.rows + kProjRows - 1) / kProjRows;
+        // Two channel blocks per workgroup once the grid passes one (FP8: two)
+        // workgroups per CU, sharing its LayerNorms (400 rows, n 2400: INT8
+        // 19.8 -> 14.9, FP8 40.6 -> 34; four blocks INT8 17.5).
+        const int reps = int64_t(blocks) * tiles > (a.fmt == I8 ? 256 : 512) ? 2 : 1;
+        const dim3 grid(unsigned((blocks + reps - 1) / reps), unsigned(tiles)), block(512);
+#define QLIN_NL(F, T)                                                                           \
+    hipLaunchKernelGGL((norm_project_rows<F, T>), grid, block, 0, stream,                      \
+                       static_cast<const uint16_t *>(a.x), a.f,                                \
+                       static_cast<const uint16_t *>(a.norm_weight),                           \
+                       static_cast<const uint16_t *>(a.norm_bias), a.rows, a.k, a.eps,         \
+                       static_cast<const uint8_t *>(a.w), a.sw, a.n, reps,                     \
+                       static_cast<const uint16_t *>(a.bias), a.act,                           \
+                       static_cast<uint16_t *>(a.y), static_cast<uint16_t *>(a.normalized),   \
+                       static_cast<uint8_t *>(a.encoded), a.encoded_scales)
+        if (a.fmt == I8) { if (a.src_type == F16) QLIN_NL(I8, f16_t); else QLIN_NL(I8, bf16_t); }
+        else { if (a.src_type == F16) QLIN_NL(FP8, f16_t); else QLIN_NL(FP8, bf16_t); }
+#undef QLIN_NL
+        return;
+    }
     // Each workgroup repeats the row's LayerNorm; give it 8 * reps channels so
     // that about kTargetBlocks workgroups cover the output.
-    const int blocks8 = (a.n + 7) / 8;
     const int reps = std::max(1, std::min(kMaxReps, int((size_t(blocks8) * a.rows + kTargetBlocks - 1) / kTargetBlocks)));
     dim3 grid(unsigned((blocks8 + reps - 1) / reps), unsigned(a.rows)), block(256);
 #define QLIN_NL(F, T)                                                                           \

@@ -83,3 +83,58 @@ def test_norm_linear_per_sequence_modulation(dev, orc, fmt):
     torch.cuda.synchronize()
     assert np.array_equal(bits(normalized), nrm)
     assert np.array_equal(bits(yd), y)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fmt", [I8, FP8])
+@pytest.mark.parametrize("rows,k,n", [(1301, 4, 33), (411, 100, 129), (130, 508, 385), (1030, 512, 49)])
+def test_norm_linear_many_rows(dev, dtype, fmt, rows, k, n):
+    """Eight rows per workgroup against the one-row kernel that the same rows
+    take in calls of seven (each checked against the oracle above): every
+    output bit for bit, with partial row tiles and channel blocks, k short of
+    a 64-byte piece, several channel blocks per workgroup, every fusion, and
+    rows of zeros, infinities and NaN; operands at 2- and 4-byte alignment."""
+    from breeze_tts_cpp_amd import qlinear
+    g = torch.Generator().manual_seed(rows + k + fmt)
+    mk = lambda *s, sc=1.0, off=0.0: (off + sc * torch.randn(*s, generator=g)).to(dtype).to(dev)
+
+    def odd(t):  # the same values one element past an aligned start
+        flat = torch.empty(t.numel() + 2, dtype=t.dtype, device=dev)
+        flat[1:-1] = t.reshape(-1)
+        return flat[1:-1].view(t.shape)
+    x, res = odd(mk(rows, k, sc=2.0, off=0.3)), odd(mk(rows, k))
+    x[3], res[3] = 0, 0
+    x[8, 0], x[9, k - 1], x[rows - 1, 1] = float("inf"), float("nan"), -float("inf")
+    pb, nw, nb, b = odd(mk(k, sc=0.1)), mk(k, sc=0.1, off=1.0), odd(mk(k, sc=0.1)), odd(mk(n, sc=0.2))
+    gate, shift, scale = mk(1, k, sc=0.3, off=1.0), mk(1, k, sc=0.1), mk(1, k, sc=0.1)
+    wq, sw = qlinear.row_quantize(mk(n, k, sc=0.05), fmt)
+    flat = torch.empty(n * k + 16, dtype=torch.uint8, device=dev)
+    flat[4:4 + n * k] = wq.reshape(-1)
+    wq = flat[4:4 + n * k].view(n, k)
+
+    def call(lo, hi, fused):
+        raw, nrm = torch.empty(hi - lo, k, dtype=dtype, device=dev), torch.empty(hi - lo, k, dtype=dtype, device=dev)
+        enc = torch.empty(hi - lo, k, dtype=torch.uint8, device=dev)
+        esc = torch.empty(hi - lo, dtype=torch.float32, device=dev)
+        fusion = qlinear.norm_fusion(raw=raw, **(dict(residual=res[lo:hi], projection_bias=pb, gate=gate,
+                                                      shift=shift, scale=scale) if fused else {}))
+        y = qlinear.norm_linear(x[lo:hi], wq, sw, fmt, norm_weight=nw if fused else None,
+                                norm_bias=nb if fused else None, fusion=fusion,
+                                bias=b if fused else None, activation=int(fused), normalized=nrm,
+                                encoded=(enc, esc))
+        return raw, nrm, enc, esc, y
+    for fused in (False, True):
+        print(f"norm_linear many rows dtype={dtype} fmt={fmt} rows={rows} k={k} n={n} fused={fused}",
+              flush=True)
+        got = call(0, rows, fused)
+        parts = [call(lo, min(lo + 7, rows), fused) for lo in range(0, rows, 7)]
+        torch.cuda.synchronize()
+        for what, a, ref in zip(("raw", "normalized", "codes", "scales", "y"), got, zip(*parts)):
+            ref = torch.cat(ref)
+            if a.is_floating_point():
+                nan = torch.isnan(ref)
+                assert torch.equal(torch.isnan(a), nan), what
+                a, ref = a.masked_fill(nan, 0), ref.masked_fill(nan, 0)
+                a, ref = a.view(torch.int16 if a.element_size() == 2 else torch.int32), ref.view(
+                    torch.int16 if ref.element_size() == 2 else torch.int32)
+            assert torch.equal(a, ref), what
