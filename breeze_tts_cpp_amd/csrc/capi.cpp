@@ -268,6 +268,22 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
     // 17.4 / 31.6 (four 64x32 waves: 20.0 / 38.8; random operands).
     const bool small_group = (input_group && input_group < 128) || (weight_group && weight_group < 128);
     const long tiles_128 = long((N + 127) / 128) * ((rows + 127) / 128);
+    // K groups of 128 where 128x128 tiles leave CUs without work: the smallest
+    // of 64x32, 64x64 and 128x64 whose grid is one round (group_int8 /
+    // group_fp8, us, from 128x64 or 128x128: M = 187 o_proj 11.9 / 11.3 -> 8.5 /
+    // 7.9 and down 27.9 / 26.4 -> 17.1 / 15.8 on 64x32, qkv 12.2 / 11.6 -> 10.4 /
+    // 9.8 on 64x64; M = 431 down 27.7 / 26.5 -> 21.6 / 20.1 on 64x64; 6144x1024
+    // at M = 260 10.0 -> 7.9 on 128x64). Where 128x128 tiles just pass a round,
+    // 256x128 in one (gate_up at M = 431 30.7 / 28.4 -> 27.0 / 23.7).
+    if (grouped && !small_group) {
+        const qlin_path small[] = {{QLIN_KIND_TILED, 32, 64, 1, 4, 0},
+                                   {QLIN_KIND_TILED, 64, 64, 1, 8, 0},
+                                   {QLIN_KIND_TILED, 64, 128, 1, 8, 0}};
+        for (const qlin_path &t : small)
+            if (long((N + t.channels - 1) / t.channels) * ((rows + t.tokens - 1) / t.tokens) <= 256)
+                return t;
+        if (tiles_128 > 256 && tiles_256x128 <= 256) p.channels = 256;
+    }
     if (p.channels == 128 && p.tokens == 128 && tiles_128 <= 128 && !small_group) {
         p.tokens = 64;
         p.waves = 8;
@@ -335,10 +351,14 @@ int check_path(const qlin_path &p, int rows, int N, int K, int fmt, int input_gr
         if (p.channels == 512 || p.tokens == 512)
             return fail(QLIN_ERR_UNSUPPORTED,
                         "tiled 512-channel path is disabled (register-streamed kernel not built)");
+        // 64-channel tiles: K groups of 128 only.
+        const bool narrow = p.channels == 64 && (p.tokens == 32 || p.tokens == 64) &&
+                            (input_group || weight_group) && !(input_group && input_group < 128) &&
+                            !(weight_group && weight_group < 128);
         if (!((p.channels == 256 && (p.tokens == 256 || p.tokens == 128)) ||
-              (p.channels == 128 && (p.tokens == 128 || p.tokens == 64))))
+              (p.channels == 128 && (p.tokens == 128 || p.tokens == 64)) || narrow))
             return fail(QLIN_ERR_UNSUPPORTED,
-                        "tiled path channels x tokens must be 256x256, 256x128, 128x128 or 128x64 (got %dx%d)",
+                        "tiled path channels x tokens must be 256x256, 256x128, 128x128 or 128x64, with K groups of 128 also 64x32 or 64x64 (got %dx%d)",
                         p.channels, p.tokens);
         if (p.splits != 1)
             return fail(QLIN_ERR_UNSUPPORTED, "tiled path has no split-K variant");
@@ -348,16 +368,17 @@ int check_path(const qlin_path &p, int rows, int N, int K, int fmt, int input_gr
             return fail(QLIN_ERR_UNSUPPORTED, "tiled path has more than 2^31 - 1 macro tiles");
         // 256x256: eight waves of 128x64 (16x16 MFMA) or four of 128x128
         // (32x32 MFMA); 256x128: one workgroup of 128x64 waves (1), two waves
-        // of 128x128 (2) or eight of 128x32 (8); 128x128: four waves of 64x64
+        // of 128x128 (2) or eight of 64x64 (8); 128x128: four waves of 64x64
         // (1) or eight of 64x32 (8).
-        const bool wave_ok = (p.channels == 256 && p.tokens == 256) ? (p.waves == 8 || p.waves == 4)
+        const bool wave_ok = narrow ? p.waves == (p.tokens == 32 ? 4 : 8)
+                             : (p.channels == 256 && p.tokens == 256) ? (p.waves == 8 || p.waves == 4)
                              : (p.channels == 256 && p.tokens == 128) ? (p.waves == 1 || p.waves == 2 || p.waves == 8)
                              : p.tokens == 64 ? (p.waves == 4 || p.waves == 8)
                                               : (p.waves == 1 || p.waves == 8);
         if (!wave_ok)
             return fail(QLIN_ERR_UNSUPPORTED, "tiled %dx%d path has no %d-wave variant", p.channels,
                         p.tokens, p.waves);
-        if (p.waves != 1 && p.waves != 8 && p.tokens != 256 && p.tokens != 64 &&
+        if (p.waves != 1 && p.waves != 8 && p.tokens != 256 && p.tokens != 64 && !narrow &&
             (input_group || weight_group))
             return fail(QLIN_ERR_UNSUPPORTED, "K-group tiled path has no 32x32-tile variant");
         if ((input_group || weight_group) && p.tokens == 256)

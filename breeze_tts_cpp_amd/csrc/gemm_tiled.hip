@@ -35,8 +35,8 @@
 #include <algorithm>
 #include <type_traits>
 
-// Built twice: without (launch_tiled_plain) and with (launch_tiled_fin) the
-// fused finish epilogue; the plain build carries no finish code.
+// Built per format, without and with the fused finish epilogue; the plain
+// builds carry no finish code.
 #ifndef QLIN_FIN
 #define QLIN_FIN 0
 #endif
@@ -1299,7 +1299,7 @@ int dispatch_small_groups(const GemmArgs &a, const GemmPath &p, hipStream_t s) {
 
 // Macro tiles (weight rows x tokens) and waves per path: 256x256 with eight
 // waves of 128x64 (waves 8) or four of 128x128 on 32x32 MFMAs (wide_gemm,
-// waves 4); 256x128 with eight waves of 128x32 (8), one workgroup of four
+// waves 4); 256x128 with eight waves of 64x64 (8), one workgroup of four
 // 128x64 waves (1) or two 128x128 waves (2); 128x128 with eight waves of
 // 64x32 (8) or four of 64x64 (1).
 template <int Fmt, bool Grouped, class Out>
@@ -1336,6 +1336,15 @@ int dispatch_shape(const GemmArgs &a, const GemmPath &p, hipStream_t s) {
         // 128x64 with eight 32x32 waves, one group per 128-byte stage.
         if (p.channels == 128 && p.tokens == 64 && p.waves == 8)
             return launch_shape<Fmt, 4, 2, 2, 2, 128, 4, true, Out>(a, s);
+        // 64-channel tiles for grids that would leave CUs without work: four
+        // waves of 32x16, eight of 16x32. A group's stage costs its rescale and
+        // the LDS reads of both operands, so the time follows the tile's size
+        // (K 6144, one round, INT8: 64x32 17 us, 64x64 21.6, 128x64 25, 128x128
+        // 36); a 64x128 tile is level with 128x64.
+        if (p.channels == 64 && p.tokens == 32 && p.waves == 4)
+            return launch_shape<Fmt, 2, 2, 2, 1, 128, 6, true, Out>(a, s);
+        if (p.channels == 64 && p.tokens == 64 && p.waves == 8)
+            return launch_shape<Fmt, 4, 2, 1, 2, 128, 6, true, Out>(a, s);
         return -4;
     } else if constexpr (Fmt == I8) {
         // 256x128 with eight waves of 64x64 over 128-byte K stages (two
@@ -1426,20 +1435,20 @@ int dispatch_grouped(const GemmArgs &a, const GemmPath &p, hipStream_t s) {
 
 #ifdef QLIN_TILED_PART
 int QLIN_TILED_PART(const GemmArgs &a, const GemmPath &p, hipStream_t stream) {
-    if (a.out_type == F16) {
-        if (a.fmt == I8) return dispatch_grouped<I8, f16_t>(a, p, stream);
-        return dispatch_grouped<FP8, f16_t>(a, p, stream);
-    }
-    if (a.fmt == I8) return dispatch_grouped<I8, bf16_t>(a, p, stream);
-    return dispatch_grouped<FP8, bf16_t>(a, p, stream);
+    if (a.out_type == F16) return dispatch_grouped<QLIN_TILED_FMT, f16_t>(a, p, stream);
+    return dispatch_grouped<QLIN_TILED_FMT, bf16_t>(a, p, stream);
 }
 #else
 size_t tiled_workspace_bytes(const GemmArgs &, const GemmPath &) { return 0; }
 
-int launch_tiled_plain(const GemmArgs &, const GemmPath &, hipStream_t);
-int launch_tiled_fin(const GemmArgs &, const GemmPath &, hipStream_t);
-int launch_tiled(const GemmArgs &a, const GemmPath &p, hipStream_t stream) {
-    return (a.bias || a.act) ? launch_tiled_fin(a, p, stream) : launch_tiled_plain(a, p, stream);
+int launch_tiled_i8(const GemmArgs &, const GemmPath &, hipStream_t);
+int launch_tiled_i8_fin(const GemmArgs &, const GemmPath &, hipStream_t);
+int launch_tiled_fp8(const GemmArgs &, const GemmPath &, hipStream_t);
+int launch_tiled_fp8_fin(const GemmArgs &, const GemmPath &, hipStream_t);
+int launch_tiled(const GemmArgs &a, const GemmPath &p, hipStream_t s) {
+    const bool fin = a.bias || a.act;
+    if (a.fmt == I8) return fin ? launch_tiled_i8_fin(a, p, s) : launch_tiled_i8(a, p, s);
+    return fin ? launch_tiled_fp8_fin(a, p, s) : launch_tiled_fp8(a, p, s);
 }
 #endif
 
