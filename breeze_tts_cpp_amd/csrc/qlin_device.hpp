@@ -139,12 +139,19 @@ template <int Fmt> __device__ __forceinline__ float quant_scale(float amax) {
     return amax == 0 ? 1.f : fmaxf(amax / range, 1.17549435e-38f);
 }
 
-// Rademacher sign of the H128 rotation for an absolute column (reference
-// quant_device.cuh:166-168).
-__device__ __forceinline__ float rotation_sign(int column) {
-    uint32_t h = uint32_t(column) * 0x45d9f3bu;
-    h = (h ^ (h >> 16)) * 0x45d9f3bu;
-    return ((h ^ (h >> 16)) & 1u) ? 1.f : -1.f;
+// Rademacher signs of the H128 rotation for the absolute columns [column,
+// column + 8) (reference quant_device.cuh:166-168: with h = column * C and
+// h' = (h ^ h >> 16) * C, + where bits 0 and 16 of h' differ), as masks for
+// the sign bit. Those two bits depend on the factors' low 17 bits, so the
+// second product takes the full-rate 24-bit multiply, and h steps by C.
+__device__ __forceinline__ void rotation_signs(int column, uint32_t (&sign)[8]) {
+    constexpr uint32_t C = 0x45d9f3bu;
+    uint32_t h = uint32_t(column) * C;
+#pragma unroll
+    for (int i = 0; i < 8; ++i, h += C) {
+        const uint32_t p = ((h ^ (h >> 16)) & 0xffffffu) * (C & 0xffffffu);
+        sign[i] = ~((p << 31) ^ (p << 15)) & 0x80000000u;
+    }
 }
 
 // Value rounded to the 16-bit storage type and widened back (exact).
@@ -163,12 +170,12 @@ template <> __device__ __forceinline__ float round16<bf16_t>(float x) {
 // same function): Cody-Waite reduction x = k ln2 + r with ln2 split into a
 // 16-bit head (0x1.62e4p-1, so k * head is exact) and a tail, |r| <= 0.347;
 // e^r by its Taylor polynomial to degree 8 (next term < 2^-32 relative), in
-// Horner form with fma; the result scaled by 2^k in two exact power-of-two
-// factors so that only the final product rounds (subnormal results included).
-// inf above 89, 0 below -104, NaN kept.
-__device__ __forceinline__ float qexp(float x) {
-    if (x != x) return x;
-    x = fminf(fmaxf(x, -104.f), 89.f);
+// Horner form with fma; the result scaled by 2^k with v_ldexp_f32, which
+// rounds once (subnormal results included). inf above 89, 0 below -104, NaN
+// kept. (Two power-of-two factors built from k, and a clamp in two
+// instructions, took eleven more instructions for the same bits of every x.)
+__device__ __forceinline__ float qexp(float x0) {
+    const float x = __builtin_amdgcn_fmed3f(x0, -104.f, 89.f);
     const float k = rintf(x * 0x1.715476p+0f);
     float r = __builtin_fmaf(-k, 0x1.62e4p-1f, x);
     r = __builtin_fmaf(-k, 0x1.7f7d1cp-20f, r);
@@ -181,9 +188,20 @@ __device__ __forceinline__ float qexp(float x) {
     p = __builtin_fmaf(p, r, 0.5f);
     p = __builtin_fmaf(p, r, 1.f);
     p = __builtin_fmaf(p, r, 1.f);
-    const int ki = int(k), k1 = ki / 2, k2 = ki - k1;
-    return (p * __uint_as_float(uint32_t(k1 + 127) << 23)) *
-           __uint_as_float(uint32_t(k2 + 127) << 23);
+    const float e = __builtin_amdgcn_ldexpf(p, int(k));
+    return x0 == x0 ? e : x0;
+}
+
+// n / d, correctly rounded, for d in [2^-16, 2^112] (or inf) and n for which
+// neither the quotient nor the products below leave the normal range: the
+// hardware reciprocal with one Newton step, the quotient and one correction
+// by its exact remainder. Half of the general division's instructions, which
+// also scales both operands for the ranges excluded here.
+__device__ __forceinline__ float quotient(float n, float d) {
+    float r = __builtin_amdgcn_rcpf(d);
+    r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+    const float q = n * r;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
 }
 
 // This library's tanh: the odd Taylor series to degree 15 for |y| < 0.5
@@ -204,7 +222,7 @@ __device__ __forceinline__ float qtanh(float y) {
         p = __builtin_fmaf(p, s, -0x1.555556p-2f);
         t = __builtin_fmaf(a * s, p, a);
     } else if (a < 9.1f) {
-        t = 1.f - 2.f / (qexp(2.f * a) + 1.f);
+        t = 1.f - quotient(2.f, qexp(2.f * a) + 1.f);
     } else {
         t = 1.f;
     }
@@ -268,10 +286,11 @@ template <int S> __device__ __forceinline__ float lane_xor(float v) {
     } else if constexpr (S == 2) {
         return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0x4E, 0xF, 0xF, false));  // [2,3,0,1]
     } else if constexpr (S == 4) {
-        // row_ror:n moves data n lanes up a 16-lane row: lane l reads l - n
-        const int from_below = __builtin_amdgcn_update_dpp(0, u, 0x124, 0xF, 0xF, false);  // l - 4
-        const int from_above = __builtin_amdgcn_update_dpp(0, u, 0x12C, 0xF, 0xF, false);  // l + 4
-        return __int_as_float((threadIdx.x & 4) ? from_below : from_above);
+        // row_ror:n moves data n lanes up a 16-lane row: lane l reads l - n.
+        // The bank mask picks the row's 4-lane banks that are written: banks
+        // 1 and 3 read l - 4, banks 0 and 2 l + 4.
+        const int odd = __builtin_amdgcn_update_dpp(0, u, 0x124, 0xF, 0xA, false);
+        return __int_as_float(__builtin_amdgcn_update_dpp(odd, u, 0x12C, 0xF, 0x5, false));
     } else if constexpr (S == 8) {
         return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0x128, 0xF, 0xF, false));  // row_ror:8
     } else {

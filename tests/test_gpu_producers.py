@@ -136,3 +136,24 @@ def test_quantized_gated_many_rows(dev, orc, width):
             torch.cuda.synchronize()
             assert np.array_equal(qd.cpu().numpy(), q)
             assert np.array_equal(sd.cpu().numpy(), sc)
+
+
+@pytest.mark.parametrize("dtype,src_type", [(torch.bfloat16, 0), (torch.float16, 5)])
+def test_quantized_gated_every_gate(dev, orc, dtype, src_type):
+    """Every finite 16-bit gate, one to a group of 32 columns (the rest are
+    zero), so that each scale holds one activation: all equal the oracle's."""
+    from breeze_tts_cpp_amd import qlinear
+    bits = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    exponent = 0x7F80 if src_type == 0 else 0x7C00
+    bits[(bits & exponent) == exponent] = 0
+    gate = np.zeros((1024, 64, 32), np.uint16)
+    gate[:, :, 0] = bits.reshape(1024, 64)
+    one = np.full((1024, 2048), 0x3F80 if src_type == 0 else 0x3C00, np.uint16)
+    inp = np.concatenate([gate.reshape(1024, 2048), one], axis=1)
+    for kind in (0, 1):
+        print(f"gated every gate dtype={dtype} kind={kind}", flush=True)
+        q, sc, _ = orc.quantized_gated(inp, kind, 4, group=32, src_type=src_type)
+        qd, sd = qlinear.quantized_gated(to_dev(inp, dtype, dev), 4, kind=kind, group=32)
+        torch.cuda.synchronize()
+        assert np.array_equal(sd.cpu().numpy(), sc)
+        assert np.array_equal(qd.cpu().numpy(), q)
