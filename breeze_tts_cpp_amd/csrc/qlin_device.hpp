@@ -149,7 +149,9 @@ __device__ __forceinline__ void rotation_signs(int column, uint32_t (&sign)[8]) 
     uint32_t h = uint32_t(column) * C;
 #pragma unroll
     for (int i = 0; i < 8; ++i, h += C) {
-        const uint32_t p = ((h ^ (h >> 16)) & 0xffffffu) * (C & 0xffffffu);
+        uint32_t p;  // (written out: of a product of masked words only two bits are
+                     // used, which the compiler takes back to the slow 32-bit form)
+        asm("v_mul_u32_u24 %0, %1, %2" : "=v"(p) : "s"(C), "v"(h ^ (h >> 16)));
         sign[i] = ~((p << 31) ^ (p << 15)) & 0x80000000u;
     }
 }
@@ -274,25 +276,24 @@ __device__ __forceinline__ int xcd_major(int i, int tiles) {
 
 // ---------------------------------------------------------------- wave64 reductions
 // The value held by lane (lane ^ S), S a power of two up to 32, without an
-// LDS round trip: S = 1, 2 by a DPP quad permutation, 4 by two row rotations
-// and a select, 8 by a row rotation, 16 / 32 by gfx950's row swaps
+// LDS round trip: S = 1, 2 by a DPP quad permutation, 4 by a quad reversal and a
+// half-row mirror, 8 by a row rotation (every lane has its source, so bound_ctrl
+// only frees the compiler to fold the exchange into the instruction that uses it), 16 / 32 by gfx950's row swaps
 // (v_permlane16_swap / v_permlane32_swap, which with both operands x leave
 // the partner's value in the first result for lanes with bit S set and in
 // the second for the others).
 template <int S> __device__ __forceinline__ float lane_xor(float v) {
     const int u = __float_as_int(v);
     if constexpr (S == 1) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0xB1, 0xF, 0xF, false));  // [1,0,3,2]
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0xB1, 0xF, 0xF, true));  // [1,0,3,2]
     } else if constexpr (S == 2) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0x4E, 0xF, 0xF, false));  // [2,3,0,1]
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0x4E, 0xF, 0xF, true));  // [2,3,0,1]
     } else if constexpr (S == 4) {
-        // row_ror:n moves data n lanes up a 16-lane row: lane l reads l - n.
-        // The bank mask picks the row's 4-lane banks that are written: banks
-        // 1 and 3 read l - 4, banks 0 and 2 l + 4.
-        const int odd = __builtin_amdgcn_update_dpp(0, u, 0x124, 0xF, 0xA, false);
-        return __int_as_float(__builtin_amdgcn_update_dpp(odd, u, 0x12C, 0xF, 0x5, false));
+        // l ^ 4 = (l ^ 3) ^ 7: the quad reversed, then the half row mirrored
+        const int r = __builtin_amdgcn_update_dpp(0, u, 0x1B, 0xF, 0xF, true);  // [3,2,1,0]
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, r, 0x141, 0xF, 0xF, true));
     } else if constexpr (S == 8) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0x128, 0xF, 0xF, false));  // row_ror:8
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0x128, 0xF, 0xF, true));  // row_ror:8
     } else {
         static_assert(S == 16 || S == 32, "lane distance");
         const auto r = S == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false)

@@ -34,11 +34,15 @@ __global__ __launch_bounds__(kThreads) void token_quantize(const uint16_t *__res
     uint8_t *dst = q + size_t(row) * cols;
     float amax = 0.f;
     if constexpr (Items > 0) {
+        uint4 raw[Items];
+#pragma unroll
+        for (int it = 0; it < Items; ++it)
+            raw[it] = load_raw8<Vec>(src, (it * kThreads + threadIdx.x) * 8, cols);
         float v[Items][8];
 #pragma unroll
         for (int it = 0; it < Items; ++it) {
             int column = (it * kThreads + threadIdx.x) * 8;
-            load8<Tin, Vec>(src, column, cols, v[it]);
+            widen8<Tin>(raw[it], v[it]);
             if constexpr (Rot) rotate8(v[it], column);
 #pragma unroll
             for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[it][i]));
