@@ -157,3 +157,23 @@ def test_quantized_gated_every_gate(dev, orc, dtype, src_type):
         torch.cuda.synchronize()
         assert np.array_equal(sd.cpu().numpy(), sc)
         assert np.array_equal(qd.cpu().numpy(), q)
+
+
+@pytest.mark.parametrize("fmt", [3, 4])
+@pytest.mark.parametrize("rows,width", [(1, 8), (3, 504), (2, 520), (5, 1016), (4, 8192), (3, 1027)])
+def test_quantized_gated_group_pieces(dev, orc, fmt, rows, width):
+    """K groups in 512-column pieces: rows that end inside a piece, inside a
+    group and on both sides of a piece's edge, and unaligned rows."""
+    from breeze_tts_cpp_amd import qlinear
+    for group, rot in ((32, 0), (64, 0), (128, 0), (128, 128)):
+        if rot and width % 128:
+            continue
+        for kind in (0, 1):
+            print(f"gated pieces fmt={fmt} {rows}x{width} group={group} rot={rot} kind={kind}", flush=True)
+            inp = rand_bits((rows, 2 * width), torch.bfloat16, width + group, 2.0)
+            q, sc, _ = orc.quantized_gated(inp, kind, fmt, group=group, rotation=rot)
+            qd, sd = qlinear.quantized_gated(to_dev(inp, torch.bfloat16, dev), fmt, kind=kind,
+                                             group=group, rotation=rot)
+            torch.cuda.synchronize()
+            assert np.array_equal(qd.cpu().numpy(), q)
+            assert np.array_equal(sd.cpu().numpy(), sc)
