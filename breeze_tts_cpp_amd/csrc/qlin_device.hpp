@@ -175,7 +175,7 @@ template <> __device__ __forceinline__ float round16<bf16_t>(float x) {
 // Horner form with fma; the result scaled by 2^k with v_ldexp_f32, which
 // rounds once (subnormal results included). inf above 89, 0 below -104, NaN
 // kept. (Two power-of-two factors built from k, and a clamp in two
-// instructions, took eleven more instructions for the same bits of every x.)
+// instructions, took nine more for the same bits of every x.)
 __device__ __forceinline__ float qexp(float x0) {
     const float x = __builtin_amdgcn_fmed3f(x0, -104.f, 89.f);
     const float k = rintf(x * 0x1.715476p+0f);
