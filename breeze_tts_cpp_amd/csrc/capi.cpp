@@ -175,13 +175,15 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
         // 4.65 us, o_proj 4.24 -> 3.64 us.
         p.waves = 8;
         p.staged = skinny_staging(rows, N, K, fmt, input_group, weight_group, p);
-        // Weight slabs of two and three blocks (K above 2048) leave no LDS for
-        // the activation tile; there the K-sliced kernel is ahead once its
+        // Where the weight slab leaves no LDS for the activation tile (two and
+        // three blocks, K above 2048) the K-sliced kernel is ahead once its
         // rows no longer fit two 16-token tiles (down among a decoder layer's
-        // other launches, FP8, M = 57: 2 us less per layer; M = 32 level).
+        // other launches, FP8, M = 57: 2 us less per layer; M = 32 level);
+        // where both fit it is behind (896 x 3584, M = 41, FP8: 4.60 us
+        // against 4.19 us).
         // With one block the slab, all of it in flight from the start, stays
         // ahead (gate_up at M = 57 2 us less per layer than K-sliced).
-        if (rows > 32 && K > 2048 && !input_group && !weight_group) {
+        if (rows > 32 && K > 2048 && p.staged != 2 && !input_group && !weight_group) {
             qlin_path sliced;
             if (sliced_tile(rows, N, K, &sliced)) return sliced;
         }

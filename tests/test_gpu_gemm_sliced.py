@@ -124,3 +124,10 @@ def test_sliced_path_validation():
     assert call(path(32, 32), ig=128, wg=128) == -4                        # per-channel only
     assert call(path(16, 16), M=1 << 30, N=1 << 30, K=16) == -4            # grid limit
     assert call(qlinear.Path(qlinear.KIND_SKINNY, 32, 32, 1, 8, 4)) == -4
+
+
+def test_decode_plan_with_room_for_both_operands():
+    """33 to 64 rows: K-sliced only where the decode kernel cannot stage the
+    activation tile beside its weight slab."""
+    assert qlinear.plan(41, 896, 3584, FP8).staged == 2
+    assert qlinear.plan(57, 2048, 6144, FP8).staged == 3
