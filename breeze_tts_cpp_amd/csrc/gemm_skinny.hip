@@ -38,19 +38,10 @@ namespace {
 constexpr bool kFin = QLIN_FIN;
 constexpr int kBlockK = 256;  // K handled per main-loop iteration (4 pieces of 64)
 
-// f(std::integral_constant<int, I>{}) for I = B .. E-1, each I a constant
-// expression in f (for per-step s_waitcnt immediates).
 // s_waitcnt vmcnt(n) leaving expcnt / lgkmcnt unconstrained (gfx9 encoding).
 template <int N> __device__ __forceinline__ void wait_vmcnt() {
     static_assert(N >= 0 && N < 64, "vmcnt range");
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-template <int B, int E, class F> __device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        static_for<B + 1, E>(f);
-    }
 }
 
 template <int Fmt> struct Mfma;

@@ -55,14 +55,6 @@ __device__ __forceinline__ void wait_lds_reads() {
 }
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
-// f(std::integral_constant<int, I>{}) for I = B .. E-1.
-template <int B, int E, class F> __device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        static_for<B + 1, E>(f);
-    }
-}
-
 template <int Fmt> struct SliceMma;
 template <> struct SliceMma<I8> {
     using Acc = i32x4;
@@ -85,11 +77,15 @@ template <> struct SliceMma<FP8> {
 // KS slices of K, WN x WM waves per slice, NF weight and MT token fragments of
 // 16 rows per wave, S stages of 128 K bytes per slice's LDS ring. `steps`
 // stages per slice; slices past K are short or empty and add zeros. WAUX: the
-// weight DMA's cache policy. `turned`: each workgroup walks its slices' stages
-// from another start. Rows of a power-of-two pitch put one K column of all
-// rows on few L2 channels, and every workgroup begins at the same columns;
-// with slices of four or more stages starting apart gains 3-7% (down at
-// M = 187 10.5 -> 9.9 us, M = 90 9.2 -> 8.9), with two stages nothing.
+// weight DMA's cache policy. `turned` (INT8, whose sums are exact in any
+// order): each workgroup walks its slices' stages from another start. Rows of
+// a power-of-two pitch put one K column of all rows on few L2 channels, and
+// every workgroup begins at the same columns; with slices of four or more
+// stages starting apart gains 3-7% (down at M = 187 10.5 -> 9.9 us, M = 90 9.2
+// -> 8.9), with two stages nothing. FP8 walks K in order: a token's fp32 sum
+// must not depend on the tile its row falls in, and starts taken from the
+// weight tile alone gain nothing (us, starts apart / in order: M = 187 9.5 /
+// 10.3, M = 431 14.2 / 14.9, but M = 57 8.5 / 7.7, 499 x 1024 x 4096 7.0 / 6.6).
 template <int Fmt, int KS, int WN, int WM, int NF, int MT, int S, int WAUX>
 __global__ __launch_bounds__(64 * KS * WN * WM, 1) void sliced_gemm(
     const uint8_t *__restrict__ x, const float *__restrict__ sx, const uint8_t *__restrict__ w,
@@ -134,7 +130,7 @@ __global__ __launch_bounds__(64 * KS * WN * WM, 1) void sliced_gemm(
     const int ks = wave / NWS, ws = wave % NWS, wn = ws % WN, wm = ws / WN;
     const int k_begin = ks * steps * BK;
     const int count = NWS > 1 ? steps : max(0, min(steps, (K - k_begin + BK - 1) / BK));
-    const int turn = turned && count > 0 ? b * 3 % count : 0;
+    const int turn = Fmt == I8 && turned && count > 0 ? b * 3 % count : 0;
     const int tiles_k = (K + 63) / 64;
     const int rows_w = min(BN, N - n_base), rows_x = min(BM, M - m_base);
     const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(

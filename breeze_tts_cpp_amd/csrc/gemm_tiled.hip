@@ -115,6 +115,17 @@ __device__ __forceinline__ void store_out16(uint16_t *dst, const uint4 &val) {
 
 constexpr int group_width(int bn, int bm) { return bn == 256 && bm == 256 ? 8 : 4; }
 
+// Sums that an FP8 tile with a turned K walk keeps (see `flip` below); with
+// one it walks K in order. As many as the registers hold: four in a 128x128
+// tile on four stages, two in a 256x128 tile (four spill), one in a 128x128
+// tile on two stages, which runs two workgroups per CU. 128x64 tiles gain 5%
+// at K = 6144 and lose 5-8% below (1024 x 2048 x 2048: 8.0 -> 8.7 us): one.
+template <int Fmt, bool Grouped, int BN, int BM, int BK, int STAGES>
+constexpr int kTurnChains = Fmt != FP8 || Grouped || BM != 128 || BK != 128 ? 1
+                            : BN == 256                                     ? 2
+                            : STAGES > 2                                    ? 4
+                                                                            : 1;
+
 template <int Fmt, int WN, int WM, int WTN, int WTM, int BK, int STAGES, bool Grouped, bool KFull,
           class Out, bool PackedW = false, int GS = 128>
 __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
@@ -224,13 +235,24 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
         uint32_t((scale_groups ? (scale_wv ? n_base : m_base) * 4 : 0) + lane * 16);
     // Per channel, the stages of each whole window of `window` (a power of
     // two) are walked from another start in each workgroup (see turn_window;
-    // 256x256 tiles carry no code for it, which cost them 1-3%).
+    // 256x256 tiles carry no code for it, which cost them 1-3%). INT8 sums are
+    // exact in any order. A token's fp32 sum must not depend on the tile its row
+    // falls in, so an FP8 window is kChains segments, and each segment's sum
+    // runs on through all windows: a tile walks segment j ^ (tm % kChains) as
+    // its j-th, and the pairwise total of the sums is the same for every tile.
+    constexpr int kChains = kTurnChains<Fmt, Grouped, BN, BM, BK, STAGES>;
     const int stages = (K + BK - 1) / BK;
+    const int segment = window / kChains;  // stages, even (or no turn)
+    const int whole = kChains > 1 && segment ? stages & -window : 0;
+    const int flip = tm % kChains * segment;
     auto issue = [&](int stage, int k0) {
         uint8_t *base = lds + (stage % STAGES) * STAGE_BYTES;
-        if constexpr (!Grouped && BM < 256)
+        if constexpr (Fmt == I8 && !Grouped && BM < 256) {
             if ((stage | (window - 1)) < stages)
                 k0 = ((stage & -window) | ((stage + 3 * b) & (window - 1))) * BK;
+        } else if constexpr (kChains > 1) {
+            if (stage < whole) k0 = (stage ^ flip) * BK;
+        }
         const bool kin = KFull || k0 + lane_chunk * 16 < K;
         const uint32_t voff = kin ? lane_voff + uint32_t(k0) : 0x80000000u;
         const uint32_t voff_p = kin ? lane_voff_p : 0x80000000u;
@@ -278,6 +300,46 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc32[i][j][e] = 0.f;
     }
+    // The sums of chains 1 .. kChains - 1 (chain 0 is acc), in walk order.
+    Acc side[kChains > 1 ? kChains - 1 : 1][kChains > 1 ? WTN : 1][kChains > 1 ? WTM : 1];
+    if constexpr (kChains > 1) {
+#pragma unroll
+        for (int c = 0; c < kChains - 1; ++c)
+#pragma unroll
+            for (int i = 0; i < WTN; ++i)
+#pragma unroll
+                for (int j = 0; j < WTM; ++j) side[c][i][j] = Acc{0, 0, 0, 0};
+    }
+    auto chain_sum = [&](auto chain, int i, int j) -> Acc & {
+        if constexpr (chain.value == 0) return acc[i][j];
+        else return side[chain.value - 1][i][j];
+    };
+    // All stages in pairs: pair(chain, s) runs stages s and s + 1 into the sum
+    // of `chain`. Returns the last stage's number where it has no partner.
+    auto walk = [&](auto pair) {
+        int s = 0;
+        if constexpr (kChains > 1) {
+            for (int w = 0; w < whole; w += window)
+                static_for<0, kChains>([&](auto chain) {
+                    for (const int end = s + segment; s < end; s += 2) pair(chain, s);
+                });
+            // Vector instructions may read an MFMA's result 12 wait states
+            // later. The compiler counts them in straight code, but has left
+            // them out where branches join.
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_nop 15");
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < WTN; ++i)
+#pragma unroll
+                for (int j = 0; j < WTM; ++j) {
+                    acc[i][j] += side[0][i][j];
+                    if constexpr (kChains == 4) acc[i][j] += side[1][i][j] + side[2][i][j];
+                }
+        }
+        for (; s + 1 < stages; s += 2) pair(std::integral_constant<int, 0>{}, s);
+        return s;
+    };
     float facc[Grouped ? WTN : 1][Grouped ? WTM : 1][4];
     if constexpr (!Grouped && !kAcc32) {
 #pragma unroll
@@ -416,20 +478,21 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
         auto read_a = [&](int st, int i) {
             return rd(lds + (st % 2) * STAGE_BYTES + a_off + i * 16 * BK, a_c0, a_c1);
         };
-        auto row = [&](int i, const i32x8 &a, const i32x8 (&bb)[WTM]) {
+        auto row = [&](auto chain, int i, const i32x8 &a, const i32x8 (&bb)[WTM]) {
 #pragma unroll
-            for (int j = 0; j < WTM; ++j) MMA::run(acc[i][j], a, bb[j]);
+            for (int j = 0; j < WTM; ++j) MMA::run(chain_sum(chain, i, j), a, bb[j]);
         };
         // Step s: weight blocks 0..WTN-2 (each reading the next block first);
         // wait for stage s+1 and barrier (every wave's reads of stage s are
         // complete: its slot takes stage s+2); read stage s+1's token
         // fragments and first weight block (unconditional: after the last
         // stage they read a slot whose values go unused); the last block.
-        auto step = [&](int s, const i32x8 (&bb)[WTM], i32x8 a, i32x8 (&nb)[WTM], i32x8 &na) {
+        auto step = [&](auto chain, int s, const i32x8 (&bb)[WTM], i32x8 a, i32x8 (&nb)[WTM],
+                        i32x8 &na) {
 #pragma unroll
             for (int i = 0; i + 1 < WTN; ++i) {
                 const i32x8 an = read_a(s, i + 1);
-                row(i, a, bb);
+                row(chain, i, a, bb);
                 a = an;
                 // Keeps the next block's reads from being hoisted (all of a
                 // stage's weight fragments at once do not fit the registers).
@@ -440,7 +503,7 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
             if (s + 2 < stages) issue(s + 2, (s + 2) * BK);
             read_b(s + 1, nb);
             na = read_a(s + 1, 0);
-            row(WTN - 1, a, bb);
+            row(chain, WTN - 1, a, bb);
         };
         i32x8 b0[WTM], b1[WTM], a0;
         wait_vmcnt<0>();
@@ -448,12 +511,11 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
         if (1 < stages) issue(1, BK);
         read_b(0, b0);
         a0 = read_a(0, 0);
-        int s = 0;
-        for (; s + 1 < stages; s += 2) {
-            step(s, b0, a0, b1, a0);
-            step(s + 1, b1, a0, b0, a0);
-        }
-        if (s < stages) step(s, b0, a0, b1, a0);
+        const int last = walk([&](auto chain, int s) {
+            step(chain, s, b0, a0, b1, a0);
+            step(chain, s + 1, b1, a0, b0, a0);
+        });
+        if (last < stages) step(std::integral_constant<int, 0>{}, last, b0, a0, b1, a0);
     } else if constexpr (!Grouped) {
         // Software pipeline, one stage per step (INT8: BK = 64, one 64-K
         // MFMA per tile, or BK = 128, two; FP8: BK = 128, one 128-K MFMA).
@@ -492,20 +554,20 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
                 }
             }
         };
-        auto mma = [&](const Frag (&a)[WTN], const Frag (&bb)[WTM], int i0, int i1) {
+        auto mma = [&](auto chain, const Frag (&a)[WTN], const Frag (&bb)[WTM], int i0, int i1) {
 #pragma unroll
             for (int i = i0; i < i1; ++i)
 #pragma unroll
-                for (int j = 0; j < WTM; ++j) MMA::run(acc[i][j], a[i], bb[j]);
+                for (int j = 0; j < WTM; ++j) MMA::run(chain_sum(chain, i, j), a[i], bb[j]);
         };
         constexpr int kEarly = WTN / 4;  // MFMA rows issued before the barrier
         // The barrier (and its lgkmcnt(0)) runs on every step, also the last:
         // with no control-flow path around it, the compiler's LDS wait
         // counting never makes a stage's MFMAs wait on the next stage's reads.
-        auto step = [&](int s, const Frag (&a)[WTN], const Frag (&bb)[WTM], Frag (&na)[WTN],
-                        Frag (&nb)[WTM]) {
+        auto step = [&](auto chain, int s, const Frag (&a)[WTN], const Frag (&bb)[WTM],
+                        Frag (&na)[WTN], Frag (&nb)[WTM]) {
             if (s + STAGES - 1 < stages) issue(s + STAGES - 1, (s + STAGES - 1) * BK);
-            mma(a, bb, 0, kEarly);
+            mma(chain, a, bb, 0, kEarly);
             if (s + STAGES - 1 < stages) wait_vmcnt<INSTS * (STAGES - 2)>();
             else if (s + 1 < stages) wait_vmcnt<0>();
             lds_barrier();
@@ -514,19 +576,18 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
             // a conditional read makes the compiler copy every one of them at
             // each stage.
             if (BK == 128 || s + 1 < stages) read(s + 1, na, nb);
-            mma(a, bb, kEarly, WTN);
+            mma(chain, a, bb, kEarly, WTN);
         };
         Frag a0[WTN], b0[WTM], a1[WTN], b1[WTM];
         if (stages >= STAGES - 1) wait_vmcnt<INSTS * (STAGES - 2)>();
         else wait_vmcnt<0>();
         lds_barrier();
         read(0, a0, b0);
-        int s = 0;
-        for (; s + 1 < stages; s += 2) {
-            step(s, a0, b0, a1, b1);
-            step(s + 1, a1, b1, a0, b0);
-        }
-        if (s < stages) step(s, a0, b0, a1, b1);
+        const int last = walk([&](auto chain, int s) {
+            step(chain, s, a0, b0, a1, b1);
+            step(chain, s + 1, a1, b1, a0, b0);
+        });
+        if (last < stages) step(std::integral_constant<int, 0>{}, last, a0, b0, a1, b1);
     } else if constexpr (GS < kGroupK) {
         // K groups of GS = 32 / 64 (the reference grouped_gemm's GroupSize,
         // the smaller of the two operands' group sizes), stage-synchronous
@@ -1247,11 +1308,14 @@ int launch_wide(const GemmArgs &a, hipStream_t stream) {
 // that start together read the same columns at the same time. Starting each
 // at another stage of a window spreads them, as long as a window of the rows
 // that an XCD's workgroups read at once stays in its L2 (4 MB; 4.5 measured
-// as well). us, in order -> turned: qkv at M = 1024 INT8 18.2 -> 14.0, FP8
-// 17.9 -> 13.8, at 730 17.2 -> 12.8; down at 4096 INT8 56.2 -> 54.5, FP8 61.6
-// -> 54.8. Not taken by 256x256 tiles (gate_up at 1024 5% slower), nor by
-// grids past one round unless all of K is one window (gate_up at M = 431 20.2
-// -> 19.4; o_proj at 4096, a window of half of K, 3% slower).
+// as well). The gain is in the weight lines: the token tiles of a column read
+// them at different times and find them in the L2 (a start taken from the
+// column alone gains nothing). us, in order -> turned: qkv at M = 1024 INT8
+// 18.2 -> 14.0, FP8 15.5 -> 12.8, at 730 17.2 -> 12.8 and 15.0 -> 12.0; down at
+// 4096 INT8 56.2 -> 54.5, FP8 60.6 -> 54.7 (two sums; 49.2 with starts as free
+// as INT8's). Not taken by 256x256 tiles (gate_up at 1024 5% slower), nor by
+// grids past one round unless all of K is one window (INT8 gate_up at M = 431
+// 20.2 -> 19.4; o_proj at 4096, a window of half of K, 3% slower).
 int turn_window(int K, int BK, int BN, int BM, int tiles_n, int tiles_m) {
     const long tiles = long(tiles_n) * tiles_m;
     const int stages = (K + BK - 1) / BK;
@@ -1273,7 +1337,8 @@ int launch_shape(const GemmArgs &a, hipStream_t stream) {
     const size_t stage = size_t(BN + BM) * BK + (Grouped && GS == 128 ? 3072 : 0);
     const size_t lds = std::max(size_t(STAGES) * stage, size_t(BN) * BM * 2) + size_t(BN + BM) * 4;
     dim3 grid(unsigned(tiles_n * tiles_m)), block(64 * WN * WM);
-    const int window = turn_window(a.K, BK, BN, BM, tiles_n, tiles_m);
+    int window = turn_window(a.K, BK, BN, BM, tiles_n, tiles_m);
+    if (Fmt == FP8 && window < 2 * kTurnChains<Fmt, Grouped, BN, BM, BK, STAGES>) window = 1;
 #define QLIN_TILED(KF, PW)                                                                      \
     hipLaunchKernelGGL((tiled_gemm<Fmt, WN, WM, WTN, WTM, BK, STAGES, Grouped, KF, Out, PW, GS>), \
                        grid, block, lds, stream, a.x, a.sx, a.w, a.sw, a.y, a.M, a.N, a.K,      \
@@ -1401,12 +1466,16 @@ int dispatch_shape(const GemmArgs &a, const GemmPath &p, hipStream_t s) {
             return launch_shape<Fmt, 2, 2, 8, 4, 64, 4, false, Out>(a, s);
         // 128x128: eight waves of 64x32 on the 16x16x128 FP8 MFMA over
         // 128-byte K stages (waves 8), or four 64x64 waves of 32x32x64 (1).
-        // Up to K = 2048 two double-buffered stages, two workgroups per CU
-        // (o_proj at 4096 17.8 us against 18.3 us on 256x128, qkv at 1024
-        // 11.7 us against 12.0 us on four stages); beyond, four stages (down
-        // at 1024 on 128x128: 23.5 us, against 32.5 us double-buffered).
+        // Up to K = 2048 two double-buffered stages, two workgroups per CU, for
+        // grids past one round (o_proj at 4096 17.8 us against 18.3 us on
+        // 256x128) and where K is too short to turn (below 1024); else four
+        // stages (down at 1024 on 128x128: 23.5 us, against 32.5 us
+        // double-buffered; grids of one round turn their walk: qkv at 1024 15.5
+        // us double-buffered, 12.8 here).
         if (p.channels == 128 && p.tokens == 128 && p.waves == 8) {
-            if (a.K <= 2048) return launch_shape<Fmt, 2, 4, 4, 2, 128, 2, false, Out>(a, s);
+            const long tiles = long((a.N + 127) / 128) * ((a.M + 127) / 128);
+            if (a.K < 1024 || (a.K <= 2048 && tiles > 256))
+                return launch_shape<Fmt, 2, 4, 4, 2, 128, 2, false, Out>(a, s);
             return launch_shape<Fmt, 2, 4, 4, 2, 128, 4, false, Out>(a, s);
         }
         if (p.channels == 128 && p.tokens == 128)

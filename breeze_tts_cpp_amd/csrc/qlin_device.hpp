@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace qlin {
 
 // Storage codes follow tts::Type (reference core/tensor.h:8).
@@ -262,6 +264,14 @@ __device__ __noinline__ void finish4(float (&v)[4], const uint16_t *bias, int n,
         if (act == FINISH_RELU) x = fmaxf(x, 0.f);
         else if (act == FINISH_GELU_TANH) x = gelu_tanh<true>(x);
         v[r] = x;
+    }
+}
+
+// f(std::integral_constant<int, I>{}) for I = B .. E-1.
+template <int B, int E, class F> __device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
     }
 }
 
