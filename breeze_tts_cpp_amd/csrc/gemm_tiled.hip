@@ -118,16 +118,22 @@ constexpr int group_width(int bn, int bm) { return bn == 256 && bm == 256 ? 8 : 
 // Sums that an FP8 tile with a turned K walk keeps (see `flip` below); with
 // one it walks K in order. As many as the registers hold: four in a 128x128
 // tile on four stages, two in a 256x128 tile (four spill), one in a 128x128
-// tile on two stages, which runs two workgroups per CU. 128x64 tiles gain 5%
-// at K = 6144 and lose 5-8% below (1024 x 2048 x 2048: 8.0 -> 8.7 us): one.
+// tile on two stages, which runs two workgroups per CU. 128x64 tiles with four
+// gain 5% at K = 6144 and lose 5-8% below (1024 x 2048 x 2048: 8.0 -> 8.7 us): one.
+template <int Fmt, int BN, int BM, int BK, int STAGES>
+constexpr int kTurnChains = Fmt != FP8 || BM != 128 || BK != 128 ? 1
+                            : BN == 256                          ? 2
+                            : STAGES > 2                         ? 4
+                                                                 : 1;
+// Tiles built with a turned walk besides the one in order. (A walk chosen at
+// run time costs calls that don't turn 2-5%: INT8 2509 x 2048 x 2048 16.1 -> 17.0
+// us.)
 template <int Fmt, bool Grouped, int BN, int BM, int BK, int STAGES>
-constexpr int kTurnChains = Fmt != FP8 || Grouped || BM != 128 || BK != 128 ? 1
-                            : BN == 256                                     ? 2
-                            : STAGES > 2                                    ? 4
-                                                                            : 1;
+constexpr bool kTurns = !Grouped && BK == 128 && BM < 256 &&
+                        (Fmt == I8 || kTurnChains<Fmt, BN, BM, BK, STAGES> > 1);
 
 template <int Fmt, int WN, int WM, int WTN, int WTM, int BK, int STAGES, bool Grouped, bool KFull,
-          class Out, bool PackedW = false, int GS = 128>
+          class Out, bool PackedW = false, int GS = 128, bool Turn = false>
 __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
     const uint8_t *__restrict__ x, const float *__restrict__ sx, const uint8_t *__restrict__ w,
     const float *__restrict__ sw, void *__restrict__ y, int M, int N, int K, int tiles_m,
@@ -240,14 +246,14 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
     // falls in, so an FP8 window is kChains segments, and each segment's sum
     // runs on through all windows: a tile walks segment j ^ (tm % kChains) as
     // its j-th, and the pairwise total of the sums is the same for every tile.
-    constexpr int kChains = kTurnChains<Fmt, Grouped, BN, BM, BK, STAGES>;
+    constexpr int kChains = Turn ? kTurnChains<Fmt, BN, BM, BK, STAGES> : 1;
     const int stages = (K + BK - 1) / BK;
-    const int segment = window / kChains;  // stages, even (or no turn)
-    const int whole = kChains > 1 && segment ? stages & -window : 0;
+    const int segment = window / kChains;  // stages, even
+    const int whole = stages & -window;
     const int flip = tm % kChains * segment;
     auto issue = [&](int stage, int k0) {
         uint8_t *base = lds + (stage % STAGES) * STAGE_BYTES;
-        if constexpr (Fmt == I8 && !Grouped && BM < 256) {
+        if constexpr (Turn && Fmt == I8) {
             if ((stage | (window - 1)) < stages)
                 k0 = ((stage & -window) | ((stage + 3 * b) & (window - 1))) * BK;
         } else if constexpr (kChains > 1) {
@@ -1310,15 +1316,24 @@ int launch_wide(const GemmArgs &a, hipStream_t stream) {
 // that an XCD's workgroups read at once stays in its L2 (4 MB; 4.5 measured
 // as well). The gain is in the weight lines: the token tiles of a column read
 // them at different times and find them in the L2 (a start taken from the
-// column alone gains nothing). us, in order -> turned: qkv at M = 1024 INT8
-// 18.2 -> 14.0, FP8 15.5 -> 12.8, at 730 17.2 -> 12.8 and 15.0 -> 12.0; down at
-// 4096 INT8 56.2 -> 54.5, FP8 60.6 -> 54.7 (two sums; 49.2 with starts as free
-// as INT8's). Not taken by 256x256 tiles (gate_up at 1024 5% slower), nor by
-// grids past one round unless all of K is one window (INT8 gate_up at M = 431
-// 20.2 -> 19.4; o_proj at 4096, a window of half of K, 3% slower).
-int turn_window(int K, int BK, int BN, int BM, int tiles_n, int tiles_m) {
+// column alone gains nothing). us, in order -> turned (weights from HBM): qkv at
+// M = 1024 INT8 15.7 -> 12.6, FP8 15.5 -> 12.8, at 730 15.2 -> 12.2 and 15.0 ->
+// 12.0; down at 2048 43 -> 35 and 32 -> 30; down at 4096 51 -> 49 and, with two
+// sums, 60.6 -> 54.7.
+// Where it lies level or behind the walk is in order (turned / in order, of 250
+// random shapes at 200 to 4096 rows):
+//  - 256x256 tiles (gate_up at 1024 5% behind) and fewer than eight stages;
+//  - past one round of workgroups, but for INT8 in two rounds with all of K in
+//    one window and no more token than weight tiles (gate_up at M = 431 20.2 ->
+//    19.4, but 2963 x 2048 x 2048 6% behind); FP8 would give up its second
+//    workgroup per CU (20-50% behind);
+//  - 128x64 tiles below K = 3584 (0.97-1.05; from there 0.83-0.90);
+//  - FP8 128x128 tiles, four stages either way above K = 2048: below K = 4608
+//    0.94-1.11, with fewer than four token tiles 0.98-1.11, else 0.89-1.03.
+int turn_window(const GemmArgs &a, int BK, int BN, int BM, int chains) {
+    const int tiles_n = (a.N + BN - 1) / BN, tiles_m = (a.M + BM - 1) / BM;
     const long tiles = long(tiles_n) * tiles_m;
-    const int stages = (K + BK - 1) / BK;
+    const int stages = (a.K + BK - 1) / BK;
     const int live = int(std::min(64L, (tiles + 7) / 8));
     const int gn = std::min(group_width(BN, BM), tiles_n);
     const int gm = std::min(tiles_m, (live + gn - 1) / gn);
@@ -1326,7 +1341,13 @@ int turn_window(int K, int BK, int BN, int BM, int tiles_n, int tiles_m) {
     const long fit = 4608L * 1024 / (rows * BK);
     int window = 1;
     while (window * 2 <= fit && window * 2 <= stages) window *= 2;
-    return BM == 256 || (tiles > 256 && window * 2 <= stages) ? 1 : window;
+    if (window < 2 * chains || stages < 8) return 1;
+    if (tiles > 256 && (a.fmt == FP8 || tiles > 512 || tiles_n < tiles_m || window < stages ||
+                        stages < 16))
+        return 1;
+    if (BM == 64 && a.K < 3584) return 1;
+    if (a.fmt == FP8 && BN == 128 && a.K > 2048 && (a.K < 4608 || tiles_m < 4)) return 1;
+    return window;
 }
 
 template <int Fmt, int WN, int WM, int WTN, int WTM, int BK, int STAGES, bool Grouped, class Out,
@@ -1337,14 +1358,23 @@ int launch_shape(const GemmArgs &a, hipStream_t stream) {
     const size_t stage = size_t(BN + BM) * BK + (Grouped && GS == 128 ? 3072 : 0);
     const size_t lds = std::max(size_t(STAGES) * stage, size_t(BN) * BM * 2) + size_t(BN + BM) * 4;
     dim3 grid(unsigned(tiles_n * tiles_m)), block(64 * WN * WM);
-    int window = turn_window(a.K, BK, BN, BM, tiles_n, tiles_m);
-    if (Fmt == FP8 && window < 2 * kTurnChains<Fmt, Grouped, BN, BM, BK, STAGES>) window = 1;
-#define QLIN_TILED(KF, PW)                                                                      \
-    hipLaunchKernelGGL((tiled_gemm<Fmt, WN, WM, WTN, WTM, BK, STAGES, Grouped, KF, Out, PW, GS>), \
-                       grid, block, lds, stream, a.x, a.sx, a.w, a.sw, a.y, a.M, a.N, a.K,      \
-                       tiles_m, tiles_n, a.input_group, a.weight_group, a.bias, a.act, window)
-    if (a.K % BK == 0) { if (a.packed) QLIN_TILED(true, true); else QLIN_TILED(true, false); }
-    else { if (a.packed) QLIN_TILED(false, true); else QLIN_TILED(false, false); }
+    const int window = kTurns<Fmt, Grouped, BN, BM, BK, STAGES>
+                           ? turn_window(a, BK, BN, BM, kTurnChains<Fmt, BN, BM, BK, STAGES>)
+                           : 1;
+#define QLIN_TILED(KF, PW, TURN)                                                                \
+    hipLaunchKernelGGL(                                                                         \
+        (tiled_gemm<Fmt, WN, WM, WTN, WTM, BK, STAGES, Grouped, KF, Out, PW, GS, TURN>), grid,  \
+        block, lds, stream, a.x, a.sx, a.w, a.sw, a.y, a.M, a.N, a.K, tiles_m, tiles_n,         \
+        a.input_group, a.weight_group, a.bias, a.act, window)
+    if constexpr (kTurns<Fmt, Grouped, BN, BM, BK, STAGES>) {
+        if (window > 1) {
+            if (a.K % BK == 0) { if (a.packed) QLIN_TILED(true, true, true); else QLIN_TILED(true, false, true); }
+            else { if (a.packed) QLIN_TILED(false, true, true); else QLIN_TILED(false, false, true); }
+            return 0;
+        }
+    }
+    if (a.K % BK == 0) { if (a.packed) QLIN_TILED(true, true, false); else QLIN_TILED(true, false, false); }
+    else { if (a.packed) QLIN_TILED(false, true, false); else QLIN_TILED(false, false, false); }
 #undef QLIN_TILED
     return 0;
 }
@@ -1473,8 +1503,7 @@ int dispatch_shape(const GemmArgs &a, const GemmPath &p, hipStream_t s) {
         // double-buffered; grids of one round turn their walk: qkv at 1024 15.5
         // us double-buffered, 12.8 here).
         if (p.channels == 128 && p.tokens == 128 && p.waves == 8) {
-            const long tiles = long((a.N + 127) / 128) * ((a.M + 127) / 128);
-            if (a.K < 1024 || (a.K <= 2048 && tiles > 256))
+            if (a.K <= 2048 && turn_window(a, 128, 128, 128, 4) == 1)
                 return launch_shape<Fmt, 2, 4, 4, 2, 128, 2, false, Out>(a, s);
             return launch_shape<Fmt, 2, 4, 4, 2, 128, 4, false, Out>(a, s);
         }
