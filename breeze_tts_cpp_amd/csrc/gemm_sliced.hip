@@ -80,12 +80,12 @@ template <> struct SliceMma<FP8> {
 // weight DMA's cache policy. `turned` (INT8, whose sums are exact in any
 // order): each workgroup walks its slices' stages from another start. Rows of
 // a power-of-two pitch put one K column of all rows on few L2 channels, and
-// every workgroup begins at the same columns; with slices of four or more
-// stages starting apart gains 3-7% (down at M = 187 10.5 -> 9.9 us, M = 90 9.2
-// -> 8.9), with two stages nothing. FP8 walks K in order: a token's fp32 sum
-// must not depend on the tile its row falls in, and starts taken from the
-// weight tile alone gain nothing (us, starts apart / in order: M = 187 9.5 /
-// 10.3, M = 431 14.2 / 14.9, but M = 57 8.5 / 7.7, 499 x 1024 x 4096 7.0 / 6.6).
+// every workgroup begins at the same columns. Tiles of 32 and more channels
+// gain 5-10% with slices of five or more stages (down at M = 187 10.3 -> 9.5 us,
+// 431 x 1536 x 4352 10.4 -> 8.5); 16-channel tiles lose 5-20% (down at M = 57 7.7 ->
+// 8.5) and slices of four stages 2-5% (499 x 1024 x 4096 6.5 -> 7.0). FP8 walks K
+// in order: a token's fp32 sum must not depend on the tile its row falls in,
+// and starts taken from the weight tile alone gain nothing.
 template <int Fmt, int KS, int WN, int WM, int NF, int MT, int S, int WAUX>
 __global__ __launch_bounds__(64 * KS * WN * WM, 1) void sliced_gemm(
     const uint8_t *__restrict__ x, const float *__restrict__ sx, const uint8_t *__restrict__ w,
@@ -378,7 +378,7 @@ int launch(const GemmArgs &a, hipStream_t stream) {
     hipLaunchKernelGGL((sliced_gemm<Fmt, KS, WN, WM, NF, MT, S, WAUX>),
                        dim3(unsigned(tiles_n * tiles_m)), dim3(64 * W), lds, stream, a.x, a.sx, a.w,
                        a.sw, a.y, a.M, a.N, a.K, tiles_m, tiles_n, steps, a.packed, a.bias, a.act,
-                       int(a.out_type == F16), int(KS == 8 && steps >= 4));
+                       int(a.out_type == F16), int(KS == 8 && BN > 16 && steps >= 5));
     return 0;
 }
 
