@@ -176,12 +176,14 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
         p.waves = 8;
         p.staged = skinny_staging(rows, N, K, fmt, input_group, weight_group, p);
         // Where the weight slab leaves no LDS for the activation tile (two and
-        // three blocks, K above 2048) the K-sliced kernel is ahead once its
-        // rows no longer fit two 16-token tiles (down among a decoder layer's
-        // other launches, FP8, M = 57: 2 us less per layer; M = 32 level);
-        // where both fit it is behind (896 x 3584, M = 41, FP8: 4.60 us
-        // against 4.19 us).
-        // With one block the slab, all of it in flight from the start, stays
+        // three blocks, K above 2048) or does not fit itself, the K-sliced kernel
+        // is ahead once its rows no longer fit two 16-token tiles: of 30 shapes at
+        // 33-64 rows, K 2304-14336, among a layer's other launches, N from 3072
+        // up takes 0.5-0.9 of the GEMM's time (14336 x 4096 at M = 57 34 -> 16 us,
+        // packed 31 -> 20), down (2048 x 6144) 1-2 us less per layer, two blocks
+        // with N up to 2048 level (-0.6 to +0.4 us). M = 32 is level; where both
+        // operands fit it is behind (896 x 3584, M = 41, FP8: 4.60 us against 4.19
+        // us). With one block the slab, all of it in flight from the start, stays
         // ahead (gate_up at M = 57 2 us less per layer than K-sliced).
         if (rows > 32 && K > 2048 && p.staged != 2 && !input_group && !weight_group) {
             qlin_path sliced;
@@ -190,12 +192,22 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
         return p;
     }
     // Up to about a thousand rows, grids that a K-sliced tile covers in one
-    // round: 65 shapes of 65-1000 rows measured 1.46x faster on average than
-    // the macro tiles below, the worst 8% slower. From 1024 rows the macro
-    // tiles fill the GPU themselves (o_proj at 1024: 9.4 us on 128x64).
+    // round: 1.4x faster on average than the macro tiles below (700 random shapes
+    // of 65-1023 rows, three of them slower, by up to 4%). The tiles of two
+    // slices give way to 128x64 macro tiles in one round where K is short: 64x96
+    // and 96x64 take 0.95-1.13 of their time below K = 1792 and 0.80-1.03 from
+    // there, 64x128 0.98-1.13 below K = 2560 and 0.80-0.99 from there (INT8 up to
+    // 1.13 where K is no multiple of 128). From 1024 rows the macro tiles fill the
+    // GPU themselves (o_proj at 1024: 9.4 us on 128x64).
     if (rows < 1024 && !input_group && !weight_group) {
         qlin_path sliced;
-        if (sliced_tile(rows, N, K, &sliced)) return sliced;
+        if (sliced_tile(rows, N, K, &sliced)) {
+            const int area = sliced.channels * sliced.tokens;
+            const int from = area == 64 * 96 ? 1792 : area == 64 * 128 ? 2560 : 0;
+            const bool macro = long((N + 127) / 128) * ((rows + 63) / 64) <= 256;
+            if (K >= from || !macro) return sliced;
+            return {QLIN_KIND_TILED, 64, 128, 1, 8, 0};
+        }
     }
     // Prefill: the macro tile by measured MI355X rules (BASELINE projections
     // at M = 1024 and 4096, per-channel and K128 groups, realistic data).
