@@ -78,6 +78,12 @@ bool skinny_stages(int rows, int N, int K, int fmt, int input_group, int weight_
     return skinny_staging(rows, N, K, fmt, input_group, weight_group, p) > 0;
 }
 
+// The K-sliced kernel addresses a tile's rows of either operand through one
+// 32-bit buffer range.
+bool sliced_range(int channels, int tokens, int K) {
+    return long(std::max(channels, tokens)) * K <= INT32_MAX;
+}
+
 // The K-sliced tile (gemm_sliced.hip) for a shape: of the tiles whose grid is
 // one round of workgroups (256 CUs), the one with the least operand bytes per
 // workgroup (they pass L2 -> LDS) plus its share of the epilogue; false when
@@ -90,7 +96,7 @@ bool sliced_tile(int rows, int N, int K, qlin_path *p) {
         const long wgs = ((long(N) + t.channels - 1) / t.channels) *
                          ((long(rows) + t.tokens - 1) / t.tokens);
         const long cost = long(K) * (t.channels + t.tokens) * 14 + t.channels * t.tokens * 243;
-        if (wgs <= 256 && cost < best) {
+        if (wgs <= 256 && cost < best && sliced_range(t.channels, t.tokens, K)) {
             best = cost;
             *p = {QLIN_KIND_SKINNY, t.tokens, t.channels, 1, 8, 3};
         }
@@ -316,6 +322,8 @@ int check_path(const qlin_path &p, int rows, int N, int K, int fmt, int input_gr
                         p.channels, p.tokens, p.waves, p.splits);
         if (input_group || weight_group)
             return fail(QLIN_ERR_UNSUPPORTED, "K-sliced paths have per-channel scales only");
+        if (!sliced_range(p.channels, p.tokens, K))
+            return fail(QLIN_ERR_UNSUPPORTED, "K-sliced tile rows exceed 2 GiB");
         if (((long(N) + p.channels - 1) / p.channels) * ((long(rows) + p.tokens - 1) / p.tokens) >
             INT32_MAX)
             return fail(QLIN_ERR_UNSUPPORTED, "K-sliced path has more than 2^31 - 1 macro tiles");

@@ -142,3 +142,20 @@ def test_two_slice_tiles_give_way():
         assert (p.kind, p.channels, p.tokens) == (qlinear.KIND_TILED, 128, 64), (M, N, K, p)
     for M, N, K in ((555, 2784, 5120), (900, 2048, 6144), (700, 2048, 2048), (187, 12288, 2048)):
         assert qlinear.plan(M, N, K, FP8).staged == 3, (M, N, K)
+
+
+def test_sliced_plan_operand_range():
+    """A K-sliced tile's rows of an operand stay below 2 GiB (32-bit buffer
+    ranges): FP8 shapes with a K past that keep the plans they had, which
+    address rows by 64 bits (33-64 rows), and a saved path is refused."""
+    for K in (1 << 25, (1 << 27) + 16, 1 << 30):
+        for M, N in ((64, 4096), (64, 16), (33, 1024), (187, 2048)):
+            p = qlinear.plan(M, N, K, FP8)
+            assert p.staged != 3 or max(p.channels, p.tokens) * K < 1 << 31, (M, N, K, p)
+    assert qlinear.plan(64, 4096, 1 << 27, FP8).staged == 0
+    assert qlinear.plan(64, 4096, 1 << 25, FP8).staged == 3  # 32 x 32 rows, 1 GiB
+    L = qlinear.load()
+    import ctypes
+    fake = 1 << 20
+    assert L.qlin_gemm(ctypes.byref(path(32, 32).to_c()), fake, fake, fake, fake, fake, 64, 64,
+                       1 << 26, FP8, BF16, 0, 0, None, 0, None) == -4
