@@ -155,7 +155,17 @@ __global__ __launch_bounds__(NT)
     }
     float v[Items][8];
 #pragma unroll
-    for (int it = 0; it < Items; ++it) gated8<T>(raw_gate[it], raw_up[it], kind, v[it]);
+    for (int it = 0; it < Items; ++it) {
+        // Of a narrow row's workgroup, waves past its end have nothing to
+        // activate (3967 rows of 128, GeLU: 11.7 us when they do, 6.9 so; 1871
+        // rows of 1024 7.8 -> 6.2).
+        if (Items > 1 || int(threadIdx.x) * 8 < width) {
+            gated8<T>(raw_gate[it], raw_up[it], kind, v[it]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[it][i] = 0.f;
+        }
+    }
     encode_row<Fmt, Items, Vec, NT>(v, q, scales, row, rows, width, 0, rot);
 }
 
