@@ -523,14 +523,23 @@ __global__ __launch_bounds__(kThreads) void pointwise_quantize(
     if (q) encode_row<Fmt, Items, Vec>(v, q, scales, row, rows, cols, group, rot);
 }
 
-// Rows of any length in 2048-column chunks: per-token scales take an amax
-// pass before the pass that writes codes, raw and retained rows (so that
-// those may alias the inputs); K-group scales need the one pass only.
+// Rows of any length in 2048-column chunks; K-group scales need one pass.
+// Per-token scales need the row's maximum before its codes: up to kHeldChunks
+// chunks the row waits for it in LDS as 16-bit values (`held`, which it is
+// rounded to; every thread reads back its own columns), longer rows take an
+// amax pass and evaluate the epilogue again in the pass that writes codes, raw
+// and retained rows (so that those may alias the inputs). Rows past two chunks
+// were held as fp32 values before, in scratch memory, since a loop of eight
+// epilogues is not unrolled, and took longer the more waves shared it (2012
+// rows of 9856 columns, FP8: 94 us with six waves per SIMD, 114 with seven, 21
+// here; two rows 18-20 -> 11).
+[[maybe_unused]] constexpr int kHeldChunks = 8;
 template <int Fmt, class T, bool Vec>
 __global__ __launch_bounds__(kThreads) void pointwise_quantize_long(
     const uint16_t *__restrict__ x, int x_rows, qlin_epilogue e, uint16_t *retained, int rows,
-    int cols, uint8_t *__restrict__ q, float *__restrict__ scales, int group, int rot) {
+    int cols, uint8_t *__restrict__ q, float *__restrict__ scales, int group, int rot, int hold) {
     __shared__ float red[8];
+    extern __shared__ uint4 held[];
     const int row = blockIdx.x, t = threadIdx.x;
     const PointwiseRow<T, Vec> r(x, x_rows, e, row, cols);
     uint16_t *kept = retained ? retained + size_t(row) * cols : nullptr;
@@ -552,7 +561,12 @@ __global__ __launch_bounds__(kThreads) void pointwise_quantize_long(
         for (int ch = 0; ch < chunks; ++ch) {
             const int column = (ch * kThreads + t) * 8;
             float v[8];
-            r.value8(column, v, false);
+            r.value8(column, v, hold);
+            if (hold) {
+                if (kept) store16x8<T, Vec>(kept, column, cols, v);
+                held[ch * kThreads + t] = uint4{pack2(v[0], v[1], T{}), pack2(v[2], v[3], T{}),
+                                                pack2(v[4], v[5], T{}), pack2(v[6], v[7], T{})};
+            }
             if (rot) rotate8(v, column);
 #pragma unroll
             for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
@@ -564,8 +578,12 @@ __global__ __launch_bounds__(kThreads) void pointwise_quantize_long(
     for (int ch = 0; ch < chunks; ++ch) {
         const int column = (ch * kThreads + t) * 8;
         float v[8];
-        r.value8(column, v, true);
-        if (kept) store16x8<T, Vec>(kept, column, cols, v);
+        if (hold) {
+            widen8<T>(held[ch * kThreads + t], v);
+        } else {
+            r.value8(column, v, true);
+            if (kept) store16x8<T, Vec>(kept, column, cols, v);
+        }
         if (rot) rotate8(v, column);
         if (group) encode_group8<Fmt, Vec>(v, dst, scales, row, rows, cols, column, group);
         else store8<Fmt, Vec>(dst, column, cols, v, inverse);
@@ -1003,20 +1021,24 @@ void launch_one(const PointwiseQuantizeArgs &a, hipStream_t s) {
     auto *x = static_cast<const uint16_t *>(a.x);
     auto *kept = static_cast<uint16_t *>(a.retained);
     auto *q = static_cast<uint8_t *>(a.values);
-    if constexpr (Items == 0)
-        hipLaunchKernelGGL((pointwise_quantize_long<Fmt, T, Vec>), dim3(a.rows), dim3(kThreads), 0,
-                           s, x, a.x_rows, a.e, kept, a.rows, a.cols, q, a.scales, a.group, rot);
-    else
+    if constexpr (Items == 0) {
+        const int chunks = (a.cols + kChunk - 1) / kChunk;
+        const bool hold = q && !a.group && chunks <= kHeldChunks;
+        hipLaunchKernelGGL((pointwise_quantize_long<Fmt, T, Vec>), dim3(a.rows), dim3(kThreads),
+                           hold ? chunks * kThreads * sizeof(uint4) : 0, s, x, a.x_rows, a.e, kept,
+                           a.rows, a.cols, q, a.scales, a.group, rot, int(hold));
+    } else
         hipLaunchKernelGGL((pointwise_quantize<Fmt, T, Items, Vec>), dim3(a.rows), dim3(kThreads),
                            0, s, x, a.x_rows, a.e, kept, a.rows, a.cols, q, a.scales, a.group, rot);
 }
 
 template <int Fmt, class T, bool Vec, class Args>
 void by_items(const Args &a, hipStream_t s) {
-    // Items: 1, 2 or 8 register-resident chunks of 2048 columns, or (0) the
-    // streaming kernel for rows longer than 16384 columns.
-    if (a.cols > 8 * kChunk) launch_one<Fmt, T, 0, Vec>(a, s);
-    else if (a.cols > 2 * kChunk) launch_one<Fmt, T, 8, Vec>(a, s);
+    // Items: 1, 2 or (LayerNorm) 8 register-resident chunks of 2048 columns, or
+    // (0) the kernel that walks the chunks of longer rows.
+    constexpr bool kPointwise = std::is_same_v<Args, PointwiseQuantizeArgs>;
+    if (a.cols > (kPointwise ? 2 : 8) * kChunk) launch_one<Fmt, T, 0, Vec>(a, s);
+    else if (!kPointwise && a.cols > 2 * kChunk) launch_one<Fmt, T, kPointwise ? 0 : 8, Vec>(a, s);
     else if (a.cols > kChunk) launch_one<Fmt, T, 2, Vec>(a, s);
     else launch_one<Fmt, T, 1, Vec>(a, s);
 }

@@ -241,3 +241,33 @@ def test_pointwise_dense(dev, orc, dtype, src_type, cols):
             qlinear.pointwise(xd, qlinear.epilogue(**dev_args), out=xd)
             torch.cuda.synchronize()
             assert np.array_equal(bits(xd), out)
+
+
+def same_values(got, want, dtype=torch.bfloat16):
+    """16-bit rows equal bit for bit, but for the payload of a NaN."""
+    a, b = (torch.from_numpy(np.ascontiguousarray(v).view(np.int16)).view(dtype) for v in (got, want))
+    nan = torch.isnan(b)
+    assert torch.equal(torch.isnan(a), nan)
+    assert np.array_equal(got[~nan.numpy()], want[~nan.numpy()])
+
+
+@pytest.mark.parametrize("fmt", [I8, FP8])
+@pytest.mark.parametrize("cols", [4096, 4097, 4104, 6144, 16383, 16384, 16385, 16392])
+def test_pointwise_quantize_held_rows(dev, orc, fmt, cols):
+    """Rows held in LDS as 16-bit values between the maximum and the codes (past
+    two chunks, up to eight), their neighbours on both sides, in place, with
+    infinities and NaN among the values."""
+    from breeze_tts_cpp_amd import qlinear
+    g = torch.Generator().manual_seed(cols)
+    x, b = mk(g, torch.bfloat16, 5, cols, sc=2.0), mk(g, torch.bfloat16, cols, sc=0.3)
+    x[1, cols - 1], x[2, 0], x[3, 4000] = 0x7F80, 0x7FC0, 0xFF80
+    for act in (0, 3, 5):
+        print(f"pointwise held fmt={fmt} cols={cols} act={act}", flush=True)
+        q, s, out, _ = orc.pointwise_quantize(x, fmt, bias=b, activation=act)
+        xd, b_d = dev16(x, torch.bfloat16, dev), dev16(b, torch.bfloat16, dev)
+        qd, sd = qlinear.pointwise_quantize(xd, fmt, qlinear.epilogue(bias=b_d, activation=act),
+                                            retained=xd)
+        torch.cuda.synchronize()
+        same_values(bits(xd), out)
+        same_codes(qd, q)
+        assert np.array_equal(sd.cpu().numpy(), s, equal_nan=True)
