@@ -108,22 +108,14 @@ __global__ __launch_bounds__(64 * KS * WN * WM, 1) void sliced_gemm(
 
     // Epilogue scales, loaded ahead of everything else.
     constexpr int PITCH = BN + 4;  // 32-bit values per row of a partial tile
-    // token tiles summed per pass: all of the tile's, or (where the partial
-    // tiles do not fit the LDS) half of each wave's
-    constexpr int TP = KS * BM * PITCH * 4 <= kRing ? MT : (MT + 1) / 2, PASSES = (MT + TP - 1) / TP;
-    constexpr int RM = TP * 16 * WM;  // rows of a pass
-    // Threads own four channels each and every kRows-th row of a pass, so
-    // a thread's weight scales are the same for all its rows.
-    constexpr int kRows = 64 * W / (BN / 4), kMaxU = (RM + kRows - 1) / kRows;
+    static_assert(KS * BM * PITCH * 4 <= kRing, "the slices' partial tiles fit the LDS");
+    // Threads own four channels each and every kRows-th row, so a thread's
+    // weight scales are the same for all its rows.
+    constexpr int kRows = 64 * W / (BN / 4), kMaxU = (BM + kRows - 1) / kRows;
     const int nl = tid % (BN / 4) * 4, r0 = tid / (BN / 4);
-    // Pass row -> tile row: wave row w holds rows [16 MT w, +16 MT).
-    auto row_of = [](int p, int r) { return (r / (TP * 16) * MT + p * TP) * 16 + r % (TP * 16); };
-    float pre_x[PASSES][kMaxU], pre_w[4];
+    float pre_x[kMaxU], pre_w[4];
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p)
-#pragma unroll
-        for (int u = 0; u < kMaxU; ++u)
-            pre_x[p][u] = sx[min(m_base + row_of(p, r0 + u * kRows), M - 1)];
+    for (int u = 0; u < kMaxU; ++u) pre_x[u] = sx[min(m_base + r0 + u * kRows, M - 1)];
 #pragma unroll
     for (int r = 0; r < 4; ++r) pre_w[r] = sw[min(n_base + nl, N - 4) + r];
 
@@ -310,51 +302,43 @@ __global__ __launch_bounds__(64 * KS * WN * WM, 1) void sliced_gemm(
     using Red = std::conditional_t<Fmt == I8, int, float>;
     typedef Red Red4 __attribute__((ext_vector_type(4)));
     Red *red = reinterpret_cast<Red *>(lds);
+    __syncthreads();
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
-        __syncthreads();
+    for (int t = 0; t < MT; ++t) {
 #pragma unroll
-        for (int tl = 0; tl < TP; ++tl) {
-            const int t = p * TP + tl;
-            if (t >= MT) break;
+        for (int f = 0; f < NF; ++f) {
+            Red4 v;
 #pragma unroll
-            for (int f = 0; f < NF; ++f) {
-                Red4 v;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = acc[f][t < MT ? t : 0][r];
-                *reinterpret_cast<Red4 *>(red + (ks * RM + (wm * TP + tl) * 16 + row16) * PITCH + (wn * NF + f) * 16 + quad * 4) = v;
-            }
+            for (int r = 0; r < 4; ++r) v[r] = acc[f][t][r];
+            *reinterpret_cast<Red4 *>(red + (ks * BM + (wm * MT + t) * 16 + row16) * PITCH + (wn * NF + f) * 16 + quad * 4) = v;
         }
-        __syncthreads();
+    }
+    __syncthreads();
 #pragma unroll
-        for (int u = 0; u < kMaxU; ++u) {
-            const int ml = r0 + u * kRows;
-            const int m = m_base + row_of(p, ml), n = n_base + nl;
-            if (r0 >= kRows || ml >= RM || (PASSES > 1 && p * TP + ml % (TP * 16) / 16 >= MT) ||
-                m >= M || n >= N)
-                continue;
-            Red4 sum = {0, 0, 0, 0};
+    for (int u = 0; u < kMaxU; ++u) {
+        const int ml = r0 + u * kRows, m = m_base + ml, n = n_base + nl;
+        if (r0 >= kRows || ml >= BM || m >= M || n >= N) continue;
+        Red4 sum = {0, 0, 0, 0};
 #pragma unroll
-            for (int q = 0; q < KS; ++q)
-                sum += *reinterpret_cast<const Red4 *>(red + (q * RM + ml) * PITCH + nl);
-            float v[4];
+        for (int q = 0; q < KS; ++q)
+            sum += *reinterpret_cast<const Red4 *>(red + (q * BM + ml) * PITCH + nl);
+        float v[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float s = float(sum[r]) * pre_x[p][u];
-                v[r] = s * pre_w[r];
-            }
-            uint2 out;
-            if (out_f16) {
-                if constexpr (kFin) finish4<f16_t>(v, bias, n, N - 1, act);
-                out.x = pack2(v[0], v[1], f16_t{});
-                out.y = pack2(v[2], v[3], f16_t{});
-            } else {
-                if constexpr (kFin) finish4<bf16_t>(v, bias, n, N - 1, act);
-                out.x = pack2(v[0], v[1], bf16_t{});
-                out.y = pack2(v[2], v[3], bf16_t{});
-            }
-            *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + size_t(m) * N + n) = out;
+        for (int r = 0; r < 4; ++r) {
+            const float s = float(sum[r]) * pre_x[u];
+            v[r] = s * pre_w[r];
         }
+        uint2 out;
+        if (out_f16) {
+            if constexpr (kFin) finish4<f16_t>(v, bias, n, N - 1, act);
+            out.x = pack2(v[0], v[1], f16_t{});
+            out.y = pack2(v[2], v[3], f16_t{});
+        } else {
+            if constexpr (kFin) finish4<bf16_t>(v, bias, n, N - 1, act);
+            out.x = pack2(v[0], v[1], bf16_t{});
+            out.y = pack2(v[2], v[3], bf16_t{});
+        }
+        *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + size_t(m) * N + n) = out;
     }
 }
 
@@ -364,14 +348,12 @@ int launch(const GemmArgs &a, hipStream_t stream) {
     // As many stages as the LDS holds; more than four measured no faster.
     constexpr int S = std::min(4, kRing / (KS * (BN + BM) * 128));
     constexpr size_t ring = size_t(KS) * S * (BN + BM) * 128;
-    constexpr size_t full = size_t(KS) * BM * (BN + 4) * 4;
-    constexpr size_t red = full <= size_t(kRing) ? full : size_t(KS) * WM * ((MT + 1) / 2 * 16) * (BN + 4) * 4;
-    constexpr size_t lds = std::max(ring, red);
+    constexpr size_t lds = std::max(ring, size_t(KS) * BM * (BN + 4) * 4);
     static_assert(lds <= size_t(kRing), "LDS");
-    // 16-channel tiles serve decode batches, whose weights pass once: the
-    // DMA's nt bit, as the decode kernel (down at M = 57 7.8 -> 7.7 us). Wider
-    // tiles' weights are read again by the other token tiles (o_proj at
-    // M = 187 5.2 us against 5.5 with the bit).
+    // 16-channel tiles carry the weight DMA's nt bit, as the decode kernel: they
+    // serve decode batches, where one token tile, seldom more, reads the weights
+    // (down at M = 57 7.8 -> 7.7 us). Wider tiles' weights are read again by the
+    // other token tiles (o_proj at M = 187 5.2 us against 5.5 with the bit).
     constexpr int WAUX = BN == 16 ? 2 : 0;
     const int tiles_n = (a.N + BN - 1) / BN, tiles_m = (a.M + BM - 1) / BM;
     const int steps = ((a.K + 127) / 128 + KS - 1) / KS;

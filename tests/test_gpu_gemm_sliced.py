@@ -22,11 +22,14 @@ def path(channels, tokens):
 
 
 # K = 16: one chunk, all slices but the first empty; 1040: a slice of one
-# stage and an empty one; 3088: stages past the ring, the last one partial;
-# 4096: slices of four whole stages (walked from different starts).
+# stage and an empty one; 3088: stages past the ring of all but the 16x16
+# tile, the last one partial; 4096: slices of four whole stages; 5264: slices
+# of six stages, past every ring, which INT8 tiles of 32 and more channels walk
+# from different starts, a slice that ends in a partial stage and an empty one.
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", [I8, FP8])
-@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (100, 112, 1040), (197, 208, 3088), (130, 96, 4096)])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (100, 112, 1040), (197, 208, 3088), (130, 96, 4096),
+                                   (130, 96, 5264)])
 def test_sliced_tiles(dev, orc, fmt, M, N, K):
     xq, sx, wq, sw = operands(orc, M, N, K, fmt, seed=M + K)
     ideal = None if fmt == I8 else orc.gemm_fp8_ideal(xq, sx, wq, sw)
