@@ -38,12 +38,6 @@ namespace {
 constexpr bool kFin = QLIN_FIN;
 constexpr int kBlockK = 256;  // K handled per main-loop iteration (4 pieces of 64)
 
-// s_waitcnt vmcnt(n) leaving expcnt / lgkmcnt unconstrained (gfx9 encoding).
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
 template <int Fmt> struct Mfma;
 template <> struct Mfma<I8> {
     using Acc = i32x4;
@@ -311,7 +305,6 @@ __global__ __launch_bounds__(64 * WK) void skinny_gemm(
     float *fq_scale = fq_amax + WK * MT * 16;
     const int slab_k0 = k_begin;
     if constexpr (SNB > 0) {
-        typedef __attribute__((address_space(3))) void *lds_ptr_t;
         if constexpr (XL) {
             // Activation rows first (L2-resident, they land before the
             // weights): each instruction moves 1 KB of consecutive (row,

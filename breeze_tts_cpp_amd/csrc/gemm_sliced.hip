@@ -44,36 +44,6 @@ namespace {
 constexpr bool kFin = QLIN_FIN;
 constexpr int kRing = int(kLdsBytes);
 
-// s_waitcnt vmcnt(n) leaving expcnt / lgkmcnt unconstrained (gfx9 encoding).
-
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-__device__ __forceinline__ void wait_lds_reads() {
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0)
-}
-typedef __attribute__((address_space(3))) void *lds_ptr_t;
-
-template <int Fmt> struct SliceMma;
-template <> struct SliceMma<I8> {
-    using Acc = i32x4;
-    // K [0, 64) of a 128-byte stage in registers 0-3, [64, 128) in 4-7.
-    __device__ static void run(Acc &c, const i32x8 &a, const i32x8 &b) {
-        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{a[0], a[1], a[2], a[3]},
-                                                  i32x4{b[0], b[1], b[2], b[3]}, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{a[4], a[5], a[6], a[7]},
-                                                  i32x4{b[4], b[5], b[6], b[7]}, c, 0, 0, 0);
-    }
-};
-template <> struct SliceMma<FP8> {
-    using Acc = f32x4;
-    // Zero scale operands: the unscaled v_mfma_f32_16x16x128_f8f6f4.
-    __device__ static void run(Acc &c, const i32x8 &a, const i32x8 &b) {
-        c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
-    }
-};
-
 // KS slices of K, WN x WM waves per slice, NF weight and MT token fragments of
 // 16 rows per wave, S stages of 128 K bytes per slice's LDS ring. `steps`
 // stages per slice; slices past K are short or empty and add zeros. WAUX: the
@@ -91,7 +61,7 @@ __global__ __launch_bounds__(64 * KS * WN * WM, 1) void sliced_gemm(
     const uint8_t *__restrict__ x, const float *__restrict__ sx, const uint8_t *__restrict__ w,
     const float *__restrict__ sw, void *__restrict__ y, int M, int N, int K, int tiles_m,
     int tiles_n, int steps, int packed, const uint16_t *__restrict__ bias, int act, int out_f16, int turned) {
-    using Mma = SliceMma<Fmt>;
+    using Mma = TileMma<Fmt>;
     using Acc = typename Mma::Acc;
     constexpr int NWS = WN * WM, W = KS * NWS;
     constexpr int BN = 16 * NF * WN, BM = 16 * MT * WM, BK = 128;

@@ -46,38 +46,10 @@ namespace {
 
 constexpr bool kFin = QLIN_FIN;
 
-template <int Fmt> struct TileMma;
-template <> struct TileMma<I8> {
-    using Acc = i32x4;
-    __device__ static void run(Acc &c, const i32x4 &a, const i32x4 &b) {
-        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
-    }
-    // A 128-byte stage: K [0, 64) in registers 0-3, [64, 128) in 4-7.
-    __device__ static void run(Acc &c, const i32x8 &a, const i32x8 &b) {
-        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{a[0], a[1], a[2], a[3]},
-                                                  i32x4{b[0], b[1], b[2], b[3]}, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{a[4], a[5], a[6], a[7]},
-                                                  i32x4{b[4], b[5], b[6], b[7]}, c, 0, 0, 0);
-    }
-};
-template <> struct TileMma<FP8> {
-    using Acc = f32x4;
-    // Zero scale operands: the unscaled v_mfma_f32_16x16x128_f8f6f4.
-    __device__ static void run(Acc &c, const i32x8 &a, const i32x8 &b) {
-        c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
-    }
-};
-
 // Physical 16-byte chunk of logical chunk c in stage row r is c ^ swizzle(r).
 template <int BK> __device__ __forceinline__ int swizzle(int r) {
     if constexpr (BK == 128) return (r >> 1) & 7;
     else return (r >> 1) & 3;
-}
-
-// s_waitcnt vmcnt(n) leaving expcnt / lgkmcnt unconstrained (gfx9 encoding).
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
 // Workgroup barrier for the LDS ring: this wave's LDS reads are complete
@@ -85,11 +57,9 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 // may be refilled after it. No memory fence: the global->LDS loads are waited
 // for explicitly with wait_vmcnt.
 __device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0)
+    wait_lds_reads();
     __builtin_amdgcn_s_barrier();
 }
-
-typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
 // Unit scales: the stage-slot scale DMA of an operand without K groups copies
 // these, so the group rescale reads its slot unconditionally (1 * s and s * 1

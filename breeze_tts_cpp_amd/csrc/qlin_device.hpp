@@ -267,6 +267,42 @@ __device__ __noinline__ void finish4(float (&v)[4], const uint16_t *bias, int n,
     }
 }
 
+// ---------------------------------------------------------------- GEMM pieces
+typedef __attribute__((address_space(3))) void *lds_ptr_t;
+
+// s_waitcnt vmcnt(n) leaving expcnt / lgkmcnt unconstrained (gfx9 encoding).
+template <int N> __device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+// s_waitcnt lgkmcnt(0) alone: this wave's LDS reads are complete.
+__device__ __forceinline__ void wait_lds_reads() {
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+}
+
+// One 16x16 tile of a stage: weights the A operand, tokens the B operand.
+template <int Fmt> struct TileMma;
+template <> struct TileMma<I8> {
+    using Acc = i32x4;
+    __device__ static void run(Acc &c, const i32x4 &a, const i32x4 &b) {
+        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
+    }
+    // A 128-byte stage: K [0, 64) in registers 0-3, [64, 128) in 4-7.
+    __device__ static void run(Acc &c, const i32x8 &a, const i32x8 &b) {
+        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{a[0], a[1], a[2], a[3]},
+                                                  i32x4{b[0], b[1], b[2], b[3]}, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{a[4], a[5], a[6], a[7]},
+                                                  i32x4{b[4], b[5], b[6], b[7]}, c, 0, 0, 0);
+    }
+};
+template <> struct TileMma<FP8> {
+    using Acc = f32x4;
+    // Zero scale operands: the unscaled v_mfma_f32_16x16x128_f8f6f4.
+    __device__ static void run(Acc &c, const i32x8 &a, const i32x8 &b) {
+        c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+    }
+};
+
 // f(std::integral_constant<int, I>{}) for I = B .. E-1.
 template <int B, int E, class F> __device__ __forceinline__ void static_for(F &&f) {
     if constexpr (B < E) {
