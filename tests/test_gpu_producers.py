@@ -177,3 +177,68 @@ def test_quantized_gated_group_pieces(dev, orc, fmt, rows, width):
             torch.cuda.synchronize()
             assert np.array_equal(qd.cpu().numpy(), q)
             assert np.array_equal(sd.cpu().numpy(), sc)
+
+
+@pytest.mark.parametrize("dtype,src_type", [(torch.bfloat16, 0), (torch.float16, 5)])
+@pytest.mark.parametrize("fmt", [3, 4])
+@pytest.mark.parametrize("width,group", [(8, 0), (9, 0), (32, 32), (33, 32), (2056, 0)])
+def test_quantized_gated_every_pattern(dev, orc, dtype, src_type, fmt, width, group):
+    """Every 16-bit pattern as a gate, and as an up value, infinities and NaN
+    included, alone in its row: both kernels (per token and K groups), vector and
+    odd widths, one and two chunks of a row."""
+    from breeze_tts_cpp_amd import qlinear
+    one = 0x3F80 if src_type == 0 else 0x3C00
+    inf = 0x7F80 if src_type == 0 else 0x7C00
+    patterns = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    if width > 64:  # the special ones and their neighbours only
+        patterns = np.concatenate([np.arange(b - 4, b + 4) & 0xFFFF for b in
+                                   (0, inf, 0x8000, inf | 0x8000, one)]).astype(np.uint16)
+    inp = np.zeros((len(patterns), 2 * width), np.uint16)
+    at = width - 1 if width % 8 else 0
+    for col, other in ((at, width + at), (width + at, at)):
+        inp[:] = 0
+        inp[:, col], inp[:, other] = patterns, one
+        for kind in (0, 1):
+            print(f"gated patterns {dtype} fmt={fmt} width={width} group={group} col={col} "
+                  f"kind={kind}", flush=True)
+            q, sc, _ = orc.quantized_gated(inp, kind, fmt, group=group, src_type=src_type)
+            qd, sd = qlinear.quantized_gated(to_dev(inp, dtype, dev), fmt, kind=kind, group=group)
+            torch.cuda.synchronize()
+            sd = sd.cpu().numpy()
+            assert np.array_equal(np.isnan(sd), np.isnan(sc))
+            assert np.array_equal(sd[~np.isnan(sc)], sc[~np.isnan(sc)])
+            assert np.array_equal(qd.cpu().numpy(), q)
+
+
+@pytest.mark.parametrize("dtype,src_type", [(torch.bfloat16, 0), (torch.float16, 5)])
+@pytest.mark.parametrize("fmt", [3, 4])
+@pytest.mark.parametrize("cols", [256, 1003])
+def test_quantized_norm_special_rows(dev, orc, dtype, src_type, fmt, cols):
+    """Residual rows with infinities and NaN, rows of zeros with eps 0 (the
+    reciprocal root of 0), squares that overflow and that vanish."""
+    from breeze_tts_cpp_amd import qlinear
+    from tests.test_gpu_quantize import special_rows
+    x = special_rows(cols, src_type)
+    w = rand_bits((cols,), dtype, cols, 0.1, 1.0)
+    u = rand_bits(x.shape, dtype, cols + 1)
+    for update in (None, u):
+        for eps in (0.0, 1e-6):
+            for group, rot in ((0, 0), (128, 128)):
+                if rot and cols % 128:
+                    continue
+                print(f"norm special {dtype} fmt={fmt} cols={cols} eps={eps} group={group} "
+                      f"update={update is not None}", flush=True)
+                res, q, sc, _ = orc.quantized_norm(x, w, fmt, update_bits=update, eps=eps,
+                                                   group=group, rotation=rot, src_type=src_type)
+                xd = to_dev(x, dtype, dev)
+                qd, sd = qlinear.quantized_norm(
+                    xd, to_dev(w, dtype, dev), fmt,
+                    update=None if update is None else to_dev(update, dtype, dev), eps=eps,
+                    group=group, rotation=rot)
+                torch.cuda.synchronize()
+                want = to_dev(res, dtype, "cpu").float()
+                assert torch.equal(xd.cpu().float().nan_to_num(nan=7.0), want.nan_to_num(nan=7.0))
+                sd = sd.cpu().numpy()
+                assert np.array_equal(np.isnan(sd), np.isnan(sc))
+                assert np.array_equal(sd[~np.isnan(sc)], sc[~np.isnan(sc)])
+                assert np.array_equal(qd.cpu().numpy(), q)

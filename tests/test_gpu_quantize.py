@@ -141,3 +141,47 @@ def test_zero_rows_and_extremes(dev, orc):
             q_ref, s_ref = orc.quantize_rows(bits, fmt, group=group, rotation=rotation)
             assert np.array_equal(s, s_ref), (fmt, group, rotation)
             assert np.array_equal(q, q_ref), (fmt, group, rotation)
+
+
+def special_rows(cols, src_type):
+    """16-bit rows with infinities, NaN, subnormals, the largest finite values
+    and zeros among ordinary values, at a row's first, last and middle columns."""
+    one, inf, top = (0x3F80, 0x7F80, 0x7F7F) if src_type == BF16 else (0x3C00, 0x7C00, 0x7BFF)
+    rng = np.random.default_rng(cols)
+    rows = np.full((12, cols), one, np.uint16) | (rng.integers(0, 2, (12, cols), np.uint16) << 15)
+    nan = inf | (0x40 if src_type == BF16 else 0x200)  # quiet
+    rows[0, 0], rows[1, cols - 1], rows[2, cols // 2] = nan, nan | 0x8000, nan
+    rows[3, 0], rows[4, cols - 1], rows[5, cols // 2] = inf, inf | 0x8000, inf
+    rows[5, cols // 3] = inf | 0x8000
+    rows[6, 1], rows[6, cols - 2] = nan, inf
+    rows[7] = nan
+    rows[8] = 0
+    rows[9] = rng.integers(0, 4, cols).astype(np.uint16)  # subnormals of the last place
+    rows[10] = top
+    rows[11] = 0x8000
+    return rows
+
+
+def same_floats(got, want):
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~np.isnan(want)], want[~np.isnan(want)])
+
+
+# Aligned rows take the 16-byte loads and packed codes, odd widths the plain
+# ones; 4096 columns take several pieces a lane, or one in a wider workgroup.
+@pytest.mark.parametrize("dtype,src_type", [(torch.bfloat16, BF16), (torch.float16, F16)])
+@pytest.mark.parametrize("fmt", [I8, FP8])
+@pytest.mark.parametrize("cols", [128, 512, 333, 4096, 20480])
+def test_special_values(dev, orc, dtype, src_type, fmt, cols):
+    """Rows with infinities and NaN: the codes and scales of the oracle, whose
+    maxima leave NaN out, in every encoding mode. (A NaN's code: INT8 -127,
+    FP8 NaN; the reference's fixtures hold none.)"""
+    bits = special_rows(cols, src_type)
+    for group, rot in ((0, 0), (0, 128), (32, 0), (64, 0), (128, 0), (128, 128)):
+        if rot and cols % 128:
+            continue
+        print(f"special fmt={fmt} cols={cols} group={group} rot={rot} {dtype}", flush=True)
+        q, s = run(dev, bits, fmt, group, rot, dtype)
+        q_ref, s_ref = orc.quantize_rows(bits, fmt, group=group, rotation=rot, src_type=src_type)
+        same_floats(s, s_ref)
+        assert np.array_equal(q, q_ref)

@@ -251,6 +251,46 @@ def same_values(got, want, dtype=torch.bfloat16):
     assert np.array_equal(got[~nan.numpy()], want[~nan.numpy()])
 
 
+@pytest.mark.parametrize("dtype,src_type", [(torch.bfloat16, BF16), (torch.float16, F16)])
+def test_activations_every_pattern(dev, orc, dtype, src_type):
+    """Every activation of every 16-bit value, infinities, NaN and subnormals
+    included."""
+    from breeze_tts_cpp_amd import qlinear
+    x = np.arange(65536, dtype=np.uint32).astype(np.uint16).reshape(32, 2048)
+    for act in range(9):
+        print(f"activation {act} {dtype} every pattern", flush=True)
+        _, _, out, _ = orc.pointwise_quantize(x, I8, activation=act, src_type=src_type)
+        y = qlinear.pointwise(dev16(x, dtype, dev), qlinear.epilogue(activation=act))
+        torch.cuda.synchronize()
+        same_values(bits(y), out, dtype)
+
+
+@pytest.mark.parametrize("dtype,src_type", [(torch.bfloat16, BF16), (torch.float16, F16)])
+@pytest.mark.parametrize("fmt", [I8, FP8])
+@pytest.mark.parametrize("cols", [256, 1003])
+def test_layer_norm_special_rows(dev, orc, dtype, src_type, fmt, cols):
+    """Rows with infinities and NaN, of one repeated value and of zeros with a tiny
+    eps, squares that overflow and that vanish."""
+    from breeze_tts_cpp_amd import qlinear
+    from tests.test_gpu_quantize import special_rows
+    x = special_rows(cols, src_type)
+    for eps in (1e-30, 1e-5):
+        for group, rot in ((0, 0), (128, 128)):
+            if rot and cols % 128:
+                continue
+            print(f"layer_norm special {dtype} fmt={fmt} cols={cols} eps={eps} group={group}",
+                  flush=True)
+            q, s, u, _ = orc.layer_norm_quantize(x, fmt, eps=eps, group=group, rotation=rot,
+                                                 src_type=src_type)
+            retained = torch.empty(x.shape, dtype=dtype, device=dev)
+            qd, sd = qlinear.layer_norm_quantize(dev16(x, dtype, dev), fmt, eps=eps,
+                                                 retained=retained, group=group, rotation=rot)
+            torch.cuda.synchronize()
+            same_values(bits(retained), u, dtype)
+            same_codes(qd, q)
+            assert np.array_equal(sd.cpu().numpy(), s, equal_nan=True)
+
+
 @pytest.mark.parametrize("fmt", [I8, FP8])
 @pytest.mark.parametrize("cols", [4096, 4097, 4104, 6144, 16383, 16384, 16385, 16392])
 def test_pointwise_quantize_held_rows(dev, orc, fmt, cols):
