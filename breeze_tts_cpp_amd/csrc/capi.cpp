@@ -222,7 +222,7 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
     //  - INT8 per-channel, all with eight waves: 256x256 (128x64 waves, two
     //    double-buffered 128-byte K stages) when
     //    it has >= 192 tiles (qkv/gate_up at 4096, gate_up at 1024); else
-    //    256x128 (128x32 waves, 128-byte K stages) for >= 256 tiles in full
+    //    256x128 (64x64 waves, 128-byte K stages) for >= 256 tiles in full
     //    rounds: down at 4096 54 us against 68 us on 128x128; else 128x128
     //    (64x32 waves): qkv
     //    at 1024 14.4 us against 19.1 us with four 64x64 waves.
@@ -230,7 +230,7 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
     //    two double-buffered 128-byte K stages) when it has >= 192 tiles
     //    (gate_up at 4096 90 us; 114 us with 64-byte stages against 116 us
     //    with four 128x128 waves; gate_up at 1024 29.3 us against 33.2 us on
-    //    128x128); else 256x128 (eight 128x32 waves, the same
+    //    128x128); else 256x128 (eight 64x64 waves, the same
     //    pipeline) for >= 256 tiles in full
     //    rounds: o_proj at 4096 27.7 us against 30.2 us with four 128x64
     //    waves on 32x32x64 and 30.4 on 128x128; else 128x128 with eight 64x32 waves on
@@ -239,7 +239,7 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
     //  (Variants timed interleaved after a warm-up, median of 5 rounds: the
     //  clock settles upward under sustained MFMA load.)
     //  - K groups (no wide-kernel variant), eight waves, both formats:
-    //    256x128 (128x32 waves) for >= 256 tiles in full rounds (gate_up at
+    //    256x128 (64x64 waves) for >= 256 tiles in full rounds (gate_up at
     //    4096: INT8 193 us against 222 us on 128x128, FP8 193 us against
     //    216 us), else 128x128 (64x32 waves): down at 1024 INT8 44 us
     //    against 80 us on 256x128. Groups of 32 / 64 follow the same rule

@@ -101,8 +101,10 @@ __global__ __launch_bounds__(kThreads) void residual_rms_quantize(
 template <int Kind> __device__ __forceinline__ float activate(float x) {
     if constexpr (Kind == 0) {
         // x is a 16-bit value, so x * 2^-16 is exact; the denominator is in
-        // [2^-16, 2^112] or inf. The fixup gives the infinities and NaN of the
-        // general division, whose bits this equals for every bf16 and f16 x.
+        // [2^-16, 2^112] or inf, and 2^-15 for the tiny gates whose numerator or
+        // quotient is subnormal, where every step is exact. The fixup gives the
+        // infinities and NaN of the general division, whose bits this equals for
+        // every bf16 and f16 x.
         // The kernel is bound by its instructions; with qexp's and the encoder's
         // shorter forms and all loads issued first 41.3 -> 33.7 us at 4096 rows of
         // width 6144, 4.4 -> 3.8 at 32 and 4.0 -> 3.4 at one.

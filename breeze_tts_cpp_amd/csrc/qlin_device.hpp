@@ -196,11 +196,13 @@ __device__ __forceinline__ float qexp(float x0) {
     return x0 == x0 ? e : x0;
 }
 
-// n / d, correctly rounded, for d in [2^-16, 2^112] (or inf) and n for which
-// neither the quotient nor the products below leave the normal range: the
-// hardware reciprocal with one Newton step, the quotient and one correction
-// by its exact remainder. Half of the general division's instructions, which
-// also scales both operands for the ranges excluded here.
+// n / d by the hardware reciprocal with one Newton step, the quotient and one
+// correction by its remainder: half of the general division's instructions,
+// which also scales both operands. That this equals the division's bits rests
+// on what v_rcp_f32 gives for the divisors, not on the steps alone, so it is
+// for the operands that were compared exhaustively on gfx950 only: qtanh's
+// 2 / d for every fp32 d in [2, 2^27], and SiLU's quotient (see activate) for
+// every fp32 x.
 __device__ __forceinline__ float quotient(float n, float d) {
     float r = __builtin_amdgcn_rcpf(d);
     r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);

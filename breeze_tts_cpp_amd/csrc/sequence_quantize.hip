@@ -1085,10 +1085,10 @@ void launch_pointwise_quantize(const PointwiseQuantizeArgs &a, hipStream_t strea
     else launch_pointwise_quantize_fp8(a, vec, stream);
 }
 
-// About 2048 workgroups (8 per CU): fewer, with more channels each, are
-// slower (rows 32, k 512, n 2048: 10.4 us at 2048, 16.4 at 512, 28 at 256),
-// because a 32-lane group's channels run one after another.
-constexpr int kTargetBlocks = 2048, kMaxReps = 16;
+// norm_project's grid: about 2048 workgroups (8 per CU). Fewer, with more
+// channels each, are slower, because a 32-lane group's channels run one after
+// another.
+constexpr int kTargetBlocks = 2048;
 void launch_norm_linear(const NormLinearArgs &a, hipStream_t stream) {
     const int blocks8 = (a.n + 7) / 8;
     // Above about 3000 (FP8: 6000) pairs of a row and eight channels, eight
@@ -1122,8 +1122,9 @@ void launch_norm_linear(const NormLinearArgs &a, hipStream_t stream) {
         return;
     }
     // Each workgroup repeats the row's LayerNorm; give it 8 * reps channels so
-    // that about kTargetBlocks workgroups cover the output.
-    const int reps = std::max(1, std::min(kMaxReps, int((size_t(blocks8) * a.rows + kTargetBlocks - 1) / kTargetBlocks)));
+    // that about kTargetBlocks workgroups cover the output (below the line
+    // above, reps is at most 2 for INT8 and 3 for FP8).
+    const int reps = std::max(1, (blocks8 * a.rows + kTargetBlocks - 1) / kTargetBlocks);
     dim3 grid(unsigned((blocks8 + reps - 1) / reps), unsigned(a.rows)), block(256);
 #define QLIN_NL(F, T)                                                                           \
     hipLaunchKernelGGL((norm_project<F, T>), grid, block, 0, stream,                           \
