@@ -220,7 +220,9 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
     const int stages = (K + BK - 1) / BK;
     const int segment = window / kChains;  // stages, even
     const int whole = stages & -window;
-    const int flip = tm % kChains * segment;
+    // Packed weights past K = 2048 keep those sums, so that they give row-major
+    // weights' bits, but visit the segments in order: see turn_window.
+    const int flip = PackedW && BN == 128 && K > 2048 ? 0 : tm % kChains * segment;
     auto issue = [&](int stage, int k0) {
         uint8_t *base = lds + (stage % STAGES) * STAGE_BYTES;
         if constexpr (Turn && Fmt == I8) {
@@ -1300,6 +1302,10 @@ int launch_wide(const GemmArgs &a, hipStream_t stream) {
 //  - 128x64 tiles below K = 3584 (0.97-1.05; from there 0.83-0.90);
 //  - FP8 128x128 tiles, four stages either way above K = 2048: below K = 4608
 //    0.94-1.11, with fewer than four token tiles 0.98-1.11, else 0.89-1.03.
+//  - packed weights, whose 16 rows of a K column lie together: INT8 only 128x128
+//    tiles of one round gain (0.80-0.98 but for small weights; 128x64 1.00-1.06,
+//    256x128 0.96-1.05, past one round 0.95-1.07), FP8 not past K = 2048 (226
+//    shapes, weights from HBM).
 int turn_window(const GemmArgs &a, int BK, int BN, int BM, int chains) {
     const int tiles_n = (a.N + BN - 1) / BN, tiles_m = (a.M + BM - 1) / BM;
     const long tiles = long(tiles_n) * tiles_m;
@@ -1317,6 +1323,7 @@ int turn_window(const GemmArgs &a, int BK, int BN, int BM, int chains) {
         return 1;
     if (BM == 64 && a.K < 3584) return 1;
     if (a.fmt == FP8 && BN == 128 && a.K > 2048 && (a.K < 4608 || tiles_m < 4)) return 1;
+    if (a.packed && a.fmt == I8 && (tiles > 256 || BN != BM)) return 1;
     return window;
 }
 
@@ -1337,9 +1344,13 @@ int launch_shape(const GemmArgs &a, hipStream_t stream) {
         block, lds, stream, a.x, a.sx, a.w, a.sw, a.y, a.M, a.N, a.K, tiles_m, tiles_n,         \
         a.input_group, a.weight_group, a.bias, a.act, window)
     if constexpr (kTurns<Fmt, Grouped, BN, BM, BK, STAGES>) {
-        if (window > 1) {
-            if (a.K % BK == 0) { if (a.packed) QLIN_TILED(true, true, true); else QLIN_TILED(true, false, true); }
-            else { if (a.packed) QLIN_TILED(false, true, true); else QLIN_TILED(false, false, true); }
+        if (window > 1 && a.packed) {
+            if constexpr (Fmt == FP8 || BN == BM) {
+                if (a.K % BK == 0) QLIN_TILED(true, true, true); else QLIN_TILED(false, true, true);
+                return 0;
+            }
+        } else if (window > 1) {
+            if (a.K % BK == 0) QLIN_TILED(true, false, true); else QLIN_TILED(false, false, true);
             return 0;
         }
     }
