@@ -104,10 +104,31 @@ bool sliced_tile(int rows, int N, int K, qlin_path *p) {
     return best != LONG_MAX;
 }
 
+// Where K is short a large K-sliced tile is behind the 128x64 macro tile of the
+// same shape: its slices have few stages or none, and all of them are summed.
+// The most 128-byte stages of K for which each tile area is behind, measured
+// where 128x64 tiles also fit one round (330 shapes, weights from HBM; K-sliced /
+// macro at the line and one or two stages past it: 48x80 1.04 and 0.97, 64x64
+// 1.07 and 0.99, 48x96 1.08 and 1.00; 64x96 up to 1.13 below it and 0.80-1.03
+// past it, 64x128 up to 1.16 and 0.80-1.01, 96x96 1.11 and 1.05, level past 48
+// stages). The macro tile reads packed weights at less than its row-major rate,
+// so there the lines lie lower; FP8 has one line, because another tile sums in
+// another order and both layouts give the same bits.
+bool short_k(const qlin_path &p, int K, bool packed_i8) {
+    constexpr struct { int area, row_major, packed; } kStages[] = {
+        {32 * 80, 1, 1}, {48 * 64, 2, 1},  {48 * 80, 3, 2},   {64 * 64, 3, 2},
+        {48 * 96, 5, 3}, {64 * 96, 13, 3}, {64 * 128, 19, 5}, {96 * 96, 11, 11}};
+    for (const auto &t : kStages)
+        if (p.channels * p.tokens == t.area)
+            return (long(K) + 127) / 128 <= (packed_i8 ? t.packed : t.row_major);
+    return false;
+}
+
 // Path selection for gfx950 (256 CUs, 8 XCDs). Decode shapes stream the
 // weights once through the skinny kernel; larger token counts use the
 // LDS-tiled MFMA GEMM.
-qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_group) {
+qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_group,
+                 bool packed = false) {
     qlin_path p{};
     if (rows <= 64) {
         // Decode: the weights are streamed once and each CU's share of them
@@ -199,19 +220,14 @@ qlin_path choose(int rows, int N, int K, int fmt, int input_group, int weight_gr
     }
     // Up to about a thousand rows, grids that a K-sliced tile covers in one
     // round: 1.4x faster on average than the macro tiles below (700 random shapes
-    // of 65-1023 rows, three of them slower, by up to 4%). The tiles of two
-    // slices give way to 128x64 macro tiles in one round where K is short: 64x96
-    // and 96x64 take 0.95-1.13 of their time below K = 1792 and 0.80-1.03 from
-    // there, 64x128 0.98-1.13 below K = 2560 and 0.80-0.99 from there (INT8 up to
-    // 1.13 where K is no multiple of 128). From 1024 rows the macro tiles fill the
-    // GPU themselves (o_proj at 1024: 9.4 us on 128x64).
+    // of 65-1023 rows, three of them slower, by up to 4%), but where K is short
+    // (short_k). From 1024 rows the macro tiles fill the GPU themselves (o_proj at
+    // 1024: 9.4 us on 128x64).
     if (rows < 1024 && !input_group && !weight_group) {
         qlin_path sliced;
         if (sliced_tile(rows, N, K, &sliced)) {
-            const int area = sliced.channels * sliced.tokens;
-            const int from = area == 64 * 96 ? 1792 : area == 64 * 128 ? 2560 : 0;
             const bool macro = long((N + 127) / 128) * ((rows + 63) / 64) <= 256;
-            if (K >= from || !macro) return sliced;
+            if (!macro || !short_k(sliced, K, packed && fmt == QLIN_I8)) return sliced;
             return {QLIN_KIND_TILED, 64, 128, 1, 8, 0};
         }
     }
@@ -513,7 +529,7 @@ int gemm_impl(const qlin_path *path, const void *x, const float *sx, const void 
     if (!aligned(y, 8)) return fail(QLIN_ERR_ALIGNMENT, "output must be 8-byte aligned");
     if (!aligned(sx, 4) || !aligned(sw, 4))
         return fail(QLIN_ERR_ALIGNMENT, "scales must be 4-byte aligned");
-    qlin_path p = path && path->kind ? *path : choose(rows, N, K, fmt, input_group, weight_group);
+    qlin_path p = path && path->kind ? *path : choose(rows, N, K, fmt, input_group, weight_group, packed);
     // Packed weights stream straight into registers: no LDS slab staging (the
     // K-sliced and prefill kernels stage them like row-major ones).
     if (packed && !(path && path->kind) && p.staged != 3) p.staged = 0;

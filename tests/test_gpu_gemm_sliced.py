@@ -136,14 +136,16 @@ def test_decode_plan_with_room_for_both_operands():
     assert qlinear.plan(57, 2048, 6144, FP8).staged == 3
 
 
-def test_two_slice_tiles_give_way():
-    """Shapes whose K-sliced tile would run two slices over a short K, and which
-    128x64 macro tiles cover in one round, take the macro tile."""
+def test_short_k_gives_way():
+    """Shapes whose K-sliced tile is large for a short K, and which 128x64 macro
+    tiles cover in one round, take the macro tile."""
     for M, N, K in ((204, 6912, 1408), (499, 4096, 1024), (900, 2048, 2048), (361, 4576, 1024),
-                    (517, 2688, 896)):
+                    (517, 2688, 896), (175, 10848, 384), (192, 8320, 1408), (517, 1856, 384),
+                    (191, 5536, 640)):
         p = qlinear.plan(M, N, K, FP8)
         assert (p.kind, p.channels, p.tokens) == (qlinear.KIND_TILED, 128, 64), (M, N, K, p)
-    for M, N, K in ((555, 2784, 5120), (900, 2048, 6144), (700, 2048, 2048), (187, 12288, 2048)):
+    for M, N, K in ((555, 2784, 5120), (900, 2048, 6144), (700, 2048, 2048), (187, 12288, 2048),
+                    (191, 5536, 768), (340, 2912, 768), (187, 2048, 128)):
         assert qlinear.plan(M, N, K, FP8).staged == 3, (M, N, K)
 
 
