@@ -127,7 +127,8 @@ size_t qlin_workspace_bytes(const qlin_path *path, int rows, int N, int K, int f
  * paths above (INT8 256x128 or 128x128, FP8 128x128); split-K and
  * packed-weight paths return QLIN_ERR_UNSUPPORTED for them. Shape rules of the reference make_plan
  * (ops/cuda/quantization.cpp:210-222): K % 16 == 0, N % 16 == 0, and for
- * INT8 K <= 131071. */
+ * INT8 K <= 131071. A row's result does not depend on its place among the
+ * call's rows (in FP8 it may on their number, which the plan goes by). */
 int qlin_gemm(const qlin_path *path, const void *x, const float *sx, const void *w,
               const float *sw, void *y, int rows, int N, int K, int fmt, int out_type,
               int input_group, int weight_group, void *workspace, size_t workspace_bytes,
@@ -198,7 +199,9 @@ int qlin_pack_weights(const void *w, int N, int K, void *packed, qlin_stream_t s
 /* qlin_gemm / qlin_linear with w in the packed layout (same scales, same
  * results bit for bit). Decode paths stream the packed tiles straight into
  * MFMA registers (no LDS staging; path.staged 1 / 2 and path.splits > 1 are
- * not supported); K-sliced and prefill paths stage them through LDS like row-major weights. */
+ * not supported); K-sliced and prefill paths stage them through LDS like
+ * row-major weights. Without a path, INT8 may take another tile than qlin_plan
+ * names for row-major weights. */
 int qlin_gemm_packed(const qlin_path *path, const void *x, const float *sx, const void *w,
                      const float *sw, void *y, int rows, int N, int K, int fmt, int out_type,
                      int input_group, int weight_group, void *workspace, size_t workspace_bytes,
