@@ -302,8 +302,9 @@ __global__ __launch_bounds__(64 * WN * WM) void tiled_gemm(
                     for (const int end = s + segment; s < end; s += 2) pair(chain, s);
                 });
             // Vector instructions may read an MFMA's result 12 wait states
-            // later. The compiler counts them in straight code, but has left
-            // them out where branches join.
+            // later. The compiler's own count is right in the present code (on
+            // every path to these reads); this keeps it so whatever it makes of
+            // the branches that join here.
             __builtin_amdgcn_sched_barrier(0);
             asm volatile("s_nop 15");
             __builtin_amdgcn_sched_barrier(0);
